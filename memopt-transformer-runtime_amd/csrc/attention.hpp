@@ -80,17 +80,24 @@ unsigned long long next_decode_tag();
 // waves' (m, l, acc[D]) held in LDS. Unsplit: writes the output row. Split:
 // writes this split's partial to the workspace with agent-scope stores
 // (they bypass the per-XCD L2s, as the splits of one (b, h) run on
-// different XCDs), waits for them, and counts its arrival on (b, h) with a
-// compare-and-swap on (tag << 8 | count): a counter left by an earlier
-// launch (other tag) or zero restarts at 1, so a workspace zeroed once needs
-// no clearing between launches (a fresh one must be zero: a stale word equal
-// to this launch's (tag << 8 | count) would stop the merge). The split that
-// brings the count to `splits` merges every
-// partial (log-sum-exp, agent-scope loads) into the output row. No
-// workgroup waits for another.
+// different XCDs), waits for them, and counts its arrival on (b, h) in a
+// counter word tag << 8 | count: an atomic max with tag << 8 turns whatever
+// an earlier launch left (smaller tags; zero at first) into count 0 and the
+// add after it counts, one round trip and no retry. (A compare-and-swap per
+// arrival, retried whenever another split got in between, cost about 2 us
+// per split: one sequence of 131072 tokens x 32 heads in 24 splits took
+// 139 us, with the add 97 us.) Two cases start elsewhere: a word above this
+// tag (an older launch replayed from a graph after newer ones, or foreign
+// data) is replaced by compare-and-swap, and a replay of the launch that
+// used the word last starts at the full count and ends at twice that, from
+// where the last split takes it back. A workspace zeroed once needs no
+// clearing between launches (a fresh one must be zero: a stale word with
+// this launch's tag would miscount). The split that completes the count
+// merges every partial (log-sum-exp, agent-scope loads) into the output
+// row. No workgroup waits for another.
 template <int D, int NW>
 __device__ __forceinline__ void decode_epilogue(const DecodeParams &p, int64_t bh, int32_t split,
-                                                const float (*s_acc)[D], const float (*s_ml)[2]) {
+                                                float (*s_acc)[D], const float (*s_ml)[2]) {
   for (int d = threadIdx.x; d < D; d += NW * 64) {
     float mx = -INFINITY;
 #pragma unroll
@@ -118,33 +125,64 @@ __device__ __forceinline__ void decode_epilogue(const DecodeParams &p, int64_t b
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partial stores are complete
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned long long *cnt = p.ws_cnt + bh;
-    unsigned long long e = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), nv;
-    do {
-      nv = (e >> 8) == p.tag ? e + 1 : (p.tag << 8) | 1;
-    } while (!__hip_atomic_compare_exchange_strong(cnt, &e, nv, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT));
-    s_last = (int)(nv & 0xFF) == p.splits;
+    unsigned long long *cnt = p.ws_cnt + bh, base = p.tag << 8;
+    // (two operations of one lane on one address: they take effect in order)
+    __hip_atomic_fetch_max(cnt, base, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    unsigned long long nv = __hip_atomic_fetch_add(cnt, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+    if (((nv - 1) >> 8) != p.tag) {  // a larger word was there
+      unsigned long long e = __hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      do {
+        nv = (e >> 8) == p.tag ? e + 1 : base | 1;
+      } while (!__hip_atomic_compare_exchange_strong(cnt, &e, nv, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT));
+    }
+    const int n = (int)(nv & 0xFF);
+    s_last = n == p.splits || n == 2 * p.splits;
+    if (n == 2 * p.splits)
+      __hip_atomic_store(cnt, base | (unsigned)p.splits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (!s_last) return;
-  const float *ml = p.ws_ml + bh * p.splits * 2;
-  for (int d = threadIdx.x; d < D; d += NW * 64) {
-    float mx = -INFINITY;
-    for (int s = 0; s < p.splits; ++s)
-      mx = fmaxf(mx, __hip_atomic_load(&ml[2 * s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    float lt = 0.0f, o = 0.0f;
-    for (int s = 0; s < p.splits; ++s) {
-      const float ms = __hip_atomic_load(&ml[2 * s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float ls = __hip_atomic_load(&ml[2 * s + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float os = __hip_atomic_load(&p.ws_o[(bh * p.splits + s) * D + d], __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-      const float f = ms == -INFINITY ? 0.0f : fast_exp2(ms - mx);
-      lt += ls * f;
-      o += os * f;
+  // The merge is two memory round trips, not two per split: every wave loads
+  // all (m, l) pairs at once (lane s takes split s; splits <= 64), and the
+  // o rows are dealt to NT / D parts of the workgroup, each with its loads
+  // issued together before any is used, the parts' sums meeting in LDS.
+  constexpr int NT = NW * 64, PARTS = NT / D, WPD = D / 64, R = 8;
+  static_assert(NT % D == 0 && PARTS <= NW, "whole parts; their sums fit s_acc's rows");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int part = wave / WPD, d = (wave % WPD) * 64 + lane;
+  const float *ml = p.ws_ml + (bh * p.splits + min(lane, p.splits - 1)) * 2;
+  float ms = __hip_atomic_load(ml, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const float ls = __hip_atomic_load(ml + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const float *orow = p.ws_o + bh * p.splits * D + d;
+  float o = 0.0f, wgt = 0.0f, lt = 0.0f;
+  for (int s0 = part; s0 < p.splits; s0 += R * PARTS) {  // wave-uniform
+    float os[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      os[r] = __hip_atomic_load(orow + (int64_t)min(s0 + r * PARTS, p.splits - 1) * D, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
+    if (s0 == part) {  // the weights, under the loads of the first rows
+      if (lane >= p.splits) ms = -INFINITY;
+      const float mx = wave_max(ms);
+      wgt = ms == -INFINITY ? 0.0f : fast_exp2(ms - mx);
+      lt = lane < p.splits ? ls * wgt : 0.0f;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) lt += shfl_xor(lt, off);
     }
-    p.out[bh * D + d] = (half_t)(lt > 0.0f ? o / lt : 0.0f);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int s = s0 + r * PARTS;
+      const float f = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wgt), min(s, 63)));
+      o += s < p.splits ? os[r] * f : 0.0f;
+    }
   }
+  s_acc[part][d] = o;  // every thread read s_acc before the barriers above
+  __syncthreads();
+  if (part != 0) return;
+#pragma unroll
+  for (int k = 1; k < PARTS; ++k) o += s_acc[k][d];
+  p.out[bh * D + d] = (half_t)(lt > 0.0f ? o / lt : 0.0f);
 }
 
 // Split count used by the INT4 decode kernel for this launch shape.
