@@ -217,8 +217,10 @@ int memopt_dynamic_sparse_attention(const void *query, int32_t batch, int32_t q_
  * With num_sink_tokens == 0, causal == 0 and an fp16 cache it computes the
  * same function as memopt_dynamic_sparse_attention.
  * `workspace` (device, >= memopt_attention_workspace_size bytes) holds the
- * decode's split-K partials and arrival counters, or the prefill's staged
- * K/V and staging flags; it may be NULL when that size is 0. A decode
+ * decode's split-K partials and arrival counters, or a multi-query call's
+ * staged K/V and staging flags or split partials; it may be NULL when that
+ * size is 0 (and for multi-query calls over token-major INT4 codes, which
+ * then run unsplit). A decode
  * (q_len == 1) workspace must be zero before its first use; later calls may
  * reuse it without clearing (each call's counters carry the call's id, so
  * what an earlier call left is never taken for its own). A multi-query
@@ -267,8 +269,8 @@ int memopt_paged_attention(const memopt_attn_desc *desc, void *stream);
  * its last 64 KiB hold the decode's arrival counters (zero at load, then
  * only ever counters) and the rest the partials or staged K/V.
  * Results are bit-identical to memopt_paged_attention's except for
- * multi-query calls whose staging does not fit: those run the in-kernel
- * staging kernel, which needs no scratch and agrees with the staged one to
+ * multi-query calls whose staged K/V or split partials do not fit: those run
+ * the in-kernel staging kernel, or fewer splits, and agree with the other to
  * within fp16 attention tolerance, not bit for bit. A decode whose partials exceed the rest
  * (B * H * splits * (head_dim + 2) * 4 + 8 * B * H bytes; splits grow only
  * while B * H is below two workgroups per CU) returns MEMOPT_ERR_INVALID. Every call on

@@ -10,8 +10,10 @@
 //   * fp16 cache, q_len == 1, pages of 16 * 2^k tokens, D in {64, 128},
 //     16-byte aligned rows -> decode_fp16 (split-K, HBM-streaming;
 //     decode_fp16.hip);
-//   * fp16 or INT4 cache, q_len >= 2, D in {64, 128}, 16-token pages ->
-//     prefill (fp16 MFMA; prefill.hip);
+//   * q_len >= 2, D in {64, 128}, pages of a multiple of 16 tokens: few
+//     queries, few query tiles, or token-major INT4 codes -> direct (fp16
+//     MFMA straight from the cache, split-K; direct.hip); other calls over
+//     fp16 pools or INT4 pages -> prefill (staged, fp16 MFMA; prefill.hip);
 //   * anything else -> generic_attention_kernel below: one wave per
 //     (b, query, head), lanes over head dims, keys visited in order with an
 //     online softmax. INT4 elements are dequantized to fp16 exactly as the
@@ -272,7 +274,12 @@ int memopt_attention_workspace_size(const memopt_attn_desc *desc, int64_t *bytes
     int32_t splits;
     return decode_workspace(*desc, &splits, bytes);
   }
-  if (desc->batch > 0 && prefill_supported(*desc)) *bytes = prefill_workspace_bytes(*desc);
+  // (INT4 pages and fp16 pools: the staged path's size, also where the direct
+  // kernel, which needs less, takes the call)
+  if (desc->batch > 0 && desc->num_heads > 0) {
+    if (prefill_supported(*desc)) *bytes = prefill_workspace_bytes(*desc);
+    else if (direct_supported(*desc)) *bytes = direct_workspace_bytes(*desc);
+  }
   return MEMOPT_OK;
 }
 
@@ -381,6 +388,7 @@ static int paged_attention(const memopt_attn_desc &d, bool unsplit_ok, void *str
     return launch_decode_fp16(p, d.batch, d.head_dim, s);
   }
 
+  if (direct_supported(d)) return launch_direct(d, W, scale * 1.4426950408889634f, s);
   if (prefill_supported(d)) return launch_prefill(d, W, scale * 1.4426950408889634f, s);
 
   GenericParams g;
@@ -445,6 +453,8 @@ int memopt_paged_attention_noalloc(const memopt_attn_desc *desc, void *stream) {
                    "paged_attention_noalloc: the split-K partials need " + std::to_string(need) +
                        " bytes, more than the " + std::to_string((long long)kNoallocDataBytes) +
                        " bytes of the static scratch they may use");
+  } else if (direct_supported(d)) {
+    need = direct_workspace_bytes(d);  // fewer splits where the partials do not all fit
   } else if (prefill_supported(d)) {
     need = prefill_workspace_bytes(d);
     if (need > kNoallocDataBytes) need = 0;  // in-kernel staging: no scratch

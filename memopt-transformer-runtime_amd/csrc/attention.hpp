@@ -201,4 +201,16 @@ bool prefill_supported(const memopt_attn_desc &d);
 int64_t prefill_workspace_bytes(const memopt_attn_desc &d);
 int launch_prefill(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hipStream_t stream);
 
+// Multi-query kernel without staging (direct.hip): calls over INT4 pages and
+// fp16 pools with few queries or few query tiles, and any number of queries
+// over token-major INT4 codes (D in {64, 128}, pages of a multiple of 16
+// tokens, aligned strides).
+bool direct_supported(const memopt_attn_desc &d);
+// Bytes of split-K partials; a call that has less room runs fewer splits.
+int64_t direct_workspace_bytes(const memopt_attn_desc &d);
+int launch_direct(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hipStream_t stream);
+
+// CUs of the current device (looked up once).
+int compute_units();
+
 }  // namespace memopt

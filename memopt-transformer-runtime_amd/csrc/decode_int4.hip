@@ -494,7 +494,7 @@ __global__ __launch_bounds__(NW * 64) void decode_int4_pages_kernel(const Decode
   decode_epilogue<D, NW>(p, (int64_t)b * p.H + h, split, s_acc, s_ml);
 }
 
-static int device_cus() {
+int compute_units() {
   static int cus = 0;
   if (cus == 0) {
     int dev = 0;
@@ -534,7 +534,7 @@ int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited) {
   // About 2 workgroups per CU; 3 when the batch has fewer (b, h) units than
   // CUs (config 5's 128 units: 6 splits measured 1.5 % faster than 4, and
   // 2, 3 or 8 slower).
-  const int64_t target_wgs = (units < device_cus() ? 3LL : 2LL) * device_cus();
+  const int64_t target_wgs = (units < compute_units() ? 3LL : 2LL) * compute_units();
   int64_t s = (target_wgs + units - 1) / units;
   // Keep at least 4 page batches per wave.
   const int64_t cap = max_pages_visited / (4LL * sh.nw * sh.u);

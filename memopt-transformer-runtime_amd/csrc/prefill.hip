@@ -1546,18 +1546,6 @@ int64_t prefill_workspace_bytes(const memopt_attn_desc &d) {
   return stage_counters_offset(d, mc) + (int64_t)d.batch * d.num_heads * 64 * 4;
 }
 
-static int prefill_device_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0;
-    hipDeviceProp_t prop;
-    if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
-      cus = prop.multiProcessorCount;
-    if (cus <= 0) cus = 256;
-  }
-  return cus;
-}
-
 // Id of a prefill call for the in-kernel staging flags: 1 .. 2^32 - 1.
 static uint32_t next_prefill_tag() {
   static std::atomic<unsigned long long> n{0};

@@ -1,0 +1,111 @@
+"""The multi-query kernel without staging (csrc/direct.hip) against the CPU
+oracle: INT4 pages, token-major codes with fp32 and fp16 scales, and fp16
+pools, at the edges of its 16-query blocks, 32-token steps and splits."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from gpu_helpers import assert_close, dev, memopt_C, to_dev
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, H, D, bs, ctx, Lq, W, sinks, causal, unlink
+    (1, 1, 64, 16, [2], 2, 64, 0, True, False),              # one partial chunk
+    (2, 2, 128, 16, [17, 1], 2, 128, 4, True, False),         # ctx < q_len: a query that sees nothing
+    (1, 2, 128, 16, [33], 15, 16, 2, True, False),            # odd chunk count, window inside one chunk
+    (2, 3, 64, 16, [700, 63], 16, 100, 4, False, True),       # non-causal window and sinks, holes
+    (1, 2, 128, 16, [1000], 17, 2048, 0, True, True),         # first size with two query blocks per wave
+    (1, 2, 64, 16, [500], 33, 40, 70, True, False),           # sinks longer than the window, third block of 1 query
+    (2, 2, 128, 48, [400, 96], 5, 512, 4, True, True),        # pages of three chunks (fp16, token-major)
+    (1, 1, 128, 32, [2049], 7, 4096, 4, True, False),         # splits, last one partly empty
+    (1, 2, 64, 16, [0], 3, 64, 4, False, False),              # empty context -> zeros
+]
+
+
+def _inputs(seed, B, H, D, bs, ctx, Lq, unlink):
+    rng = np.random.default_rng(seed)
+    M = max(1, (max(ctx) + bs - 1) // bs)
+    nb = B * M + 2
+    k = (rng.standard_normal((nb, bs, H, D)) * np.where(rng.random((nb, bs, H, D)) < 0.01, 8, 1)).astype(np.float16)
+    v = rng.standard_normal((nb, bs, H, D)).astype(np.float16)
+    q = rng.standard_normal((B, Lq, H, D)).astype(np.float16)
+    bt = rng.permutation(nb)[:B * M].reshape(B, M).astype(np.int32)
+    if unlink:
+        bt[0, M // 2] = -1
+        bt[-1, 0] = nb + 5
+    return q, k, v, bt, np.array(ctx, np.int32)
+
+
+@pytest.mark.parametrize("layout", ["pages", "rows", "rows_f16", "fp16"])
+@pytest.mark.parametrize("case", CASES)
+def test_direct_vs_oracle(case, layout):
+    B, H, D, bs, ctx, Lq, W, sinks, causal, unlink = case
+    if layout == "pages" and bs != 16:
+        bs = 16
+    q, k, v, bt, cl = _inputs(Lq * 7 + D, B, H, D, bs, ctx, Lq, unlink)
+    kw, msl = {}, 1 << 20
+    obt = np.where(bt >= k.shape[0], -1, bt).astype(np.int32)  # out-of-pool entries are skipped
+    if layout == "fp16":
+        kc, vc, kd, vd = to_dev(k), to_dev(v), k, v
+    elif layout == "pages":
+        pages = O.to_int4_pages(k, v)
+        kc = vc = to_dev(pages)
+        kd, vd = O.from_int4_pages(pages, D)
+    else:
+        (kq, ks), (vq, vs) = O.quantize_int4(k), O.quantize_int4(v)
+        if layout == "rows_f16":
+            ks, vs = ks.astype(np.float16), vs.astype(np.float16)
+        kc, vc = to_dev(kq), to_dev(vq)
+        kw = dict(key_scales=to_dev(ks), value_scales=to_dev(vs), kv_layout="token_major")
+        kd, vd = (O.dequantize_int4(c, s.astype(np.float32)) for c, s in ((kq, ks), (vq, vs)))
+    want = O.paged_attention(q, kd, vd, obt, cl, msl, W, num_sink_tokens=sinks, causal=causal)
+    got = memopt_C.dynamic_sparse_attention(to_dev(q), kc, vc, to_dev(bt), to_dev(cl), msl, W,
+                                            num_sink_tokens=sinks, causal=causal, **kw)
+    assert_close(got, want, what=f"{layout} {case}")
+    # without a workspace the call runs unsplit
+    one = memopt_C.PreparedAttention(to_dev(q), kc, vc, to_dev(bt), to_dev(cl), msl, W, num_sink_tokens=sinks,
+                                     causal=causal, no_alloc=True, **kw)
+    assert_close(one(), want, what=f"{layout} {case} no_alloc")
+
+
+def test_direct_many_splits():
+    """One (sequence, head) over 16400 tokens: 64 splits, in fp16 and both INT4 layouts."""
+    for layout in ("pages", "rows", "fp16"):
+        test_direct_vs_oracle((1, 1, 128, 16, [16400], 3, 1 << 20, 4, True, False), layout)
+    torch.cuda.synchronize(dev())
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("scale", [np.inf, np.nan, 3e4])
+def test_direct_rows_non_finite_values(D, scale):
+    """Token-major codes whose V scale is inf, NaN or large enough for fp16
+    overflow in one group of one token: queries that do not see the token
+    (causal, window) are as without it, the others get its inf or NaN in that
+    group's dims only."""
+    B, H, bs, n, Lq, W = 1, 2, 16, 200, 40, 30
+    q, k, v, bt, cl = _inputs(3, B, H, D, bs, [n], Lq, False)
+    (kq, ks), (vq, vs) = O.quantize_int4(k), O.quantize_int4(v)
+    key = n - 25                                     # seen by the queries at 175 .. 199 only
+    page, G = int(bt[0, key // bs]), D // 64
+    vs = vs.copy().reshape(-1, bs, H, G)
+    vs[page, key % bs, 1, G - 1] = scale
+    vs = vs.reshape(-1)
+    got = memopt_C.dynamic_sparse_attention(to_dev(q), to_dev(kq), to_dev(vq), to_dev(bt), to_dev(cl), n, W,
+                                            causal=True, key_scales=to_dev(ks), value_scales=to_dev(vs),
+                                            kv_layout="token_major").float().cpu().numpy()
+    with np.errstate(all="ignore"):
+        kd = O.dequantize_int4(kq, ks)[bt[0]].reshape(-1, H, D)[:n].astype(np.float64)
+        vd = O.dequantize_int4(vq, vs)[bt[0]].reshape(-1, H, D)[:n].astype(np.float64)
+        for i in range(Lq):
+            pos = n - Lq + i
+            lo = max(0, pos - W + 1)
+            for h in range(H):
+                s = kd[lo:pos + 1, h] @ q[0, i, h].astype(np.float64) / D ** 0.5
+                w = np.exp(s - s.max())
+                want = ((w / w.sum())[:, None] * vd[lo:pos + 1, h]).sum(0).astype(np.float16).astype(np.float32)
+                ok = np.isfinite(want)
+                assert ok.all() == (pos < key or h == 0)
+                assert_close(got[0, i, h][ok], want[ok], what=f"query {i} head {h}")
+                np.testing.assert_array_equal(got[0, i, h][~ok], want[~ok])
