@@ -226,15 +226,22 @@ __global__ __launch_bounds__(kThreads) void write_int4_kernel(
 }
 
 // Fused write + quantize, one wave per (group of 16 tokens, head, K or V).
-//  * Full page: when the group's 16 slots are one aligned page (slot of token
-//    t0 + i = 16 P + i), the wave builds the (page, head) block in its page
-//    layout: lane l = 8p + c quantizes tokens p and p + 8 over the dims
-//    [c*D/8, (c+1)*D/8) and stores exactly the bytes it owns, K and V codes as
-//    one 16-byte (D = 128) or 8-byte (D = 64) store each, the group scales as
-//    one 4-byte store per token pair. 64-groups span 4 (D = 128) or 8 (D = 64)
-//    lanes.
-//  * Otherwise (decode appends, ragged tails, arbitrary slots) it scatters
-//    8-element chunks like write_int4_kernel.
+//  * Full pages: where 16 consecutive tokens fill one aligned page (slot of
+//    token ts + i = 16 P + i), the wave whose group holds ts builds the (page,
+//    head) block in its page layout: lane l = 8p + c quantizes tokens ts + p
+//    and ts + p + 8 over the dims [c*D/8, (c+1)*D/8) and stores exactly the
+//    bytes it owns, K and V codes as one 16-byte (D = 128) or 8-byte (D = 64)
+//    store each, the group scales as one 4-byte store per token pair.
+//    64-groups span 4 (D = 128) or 8 (D = 64) lanes. ts need not be a multiple
+//    of 16: a batch of prompts puts each sequence's pages at its own offset
+//    (4 prompts of 6005 tokens x 32 heads, 3 of them off by 5 to 15, 498 MB:
+//    119 us when such groups scattered, now 94, or 5.3 TB/s, where the copy
+//    rate of this mix is 5.2; 6000-token prompts, all aligned, 90).
+//  * The other tokens of the group (decode appends, ragged heads and tails,
+//    arbitrary slots) scatter 8-element chunks like write_int4_kernel.
+// A wave finds both from the slots of its tokens, the 15 before and the 16
+// after, with a few scalar steps on a ballot, so all waves agree on which
+// tokens are part of a page.
 // 32-bit indexing: requires T * H * D < 2^31 (checked by the caller).
 template <int D>
 __global__ __launch_bounds__(kThreads) void write_int4_pages_kernel(
@@ -258,8 +265,8 @@ __global__ __launch_bounds__(kThreads) void write_int4_pages_kernel(
 
   // The full-page path's loads do not depend on the slots, so they are issued
   // before the slot check (rows clamped to T - 1; unused when the group
-  // scatters) and overlap its round trip: 2 x [16384, 32, 128] went from
-  // 0.80 to 0.84-0.86 of HBM.
+  // scatters, loaded again when its page starts at another token) and overlap
+  // its round trip: 2 x [16384, 32, 128] went from 0.80 to 0.84-0.86 of HBM.
   const int p = lane >> 3, c = lane & 7;
   uint4 raw[2][KW];
 #pragma unroll
@@ -269,13 +276,36 @@ __global__ __launch_bounds__(kThreads) void write_int4_pages_kernel(
 #pragma unroll
     for (int k = 0; k < KW; ++k) raw[tk][k] = *reinterpret_cast<const uint4 *>(src + o + 8 * k);
   }
-  int32_t sl = -1;
-  if (lane < 16 && t0 + lane < T) sl = slots[t0 + lane];
-  const int32_t s0 = __builtin_amdgcn_readfirstlane(sl);
-  const bool mine = lane >= 16 || sl == s0 + (int32_t)lane;
-  const bool full = __all(mine) && s0 >= 0 && (s0 & 15) == 0 && (int64_t)s0 + 16 <= n_slots;
+  // lane i: the slot of token t0 - 15 + i, i < 47
+  const int32_t tok = (int32_t)(t0 + lane) - 15;
+  const bool in = lane < 47 && tok >= 0 && tok < (int32_t)T;
+  const int32_t sl = in ? slots[tok] : -2;
+  const int32_t nxt = __shfl_down(sl, 1, 64);
+  uint64_t run = __ballot(in && lane < 46 && nxt == sl + 1);  // token i + 1 follows token i
+  run &= run >> 1;
+  run &= run >> 2;
+  run &= run >> 4;
+  run &= run >> 7;  // the 15 tokens after token i follow it
+  const uint64_t start = run & __ballot(sl >= 0 && (sl & 15) == 0 && (int64_t)sl + 16 <= n_slots);
+  const uint32_t own = (uint32_t)(start >> 15) & 0xFFFFu;  // a page starting in this group (at most one)
+  uint64_t cov = start;
+  cov |= cov << 1;
+  cov |= cov << 2;
+  cov |= cov << 4;
+  cov |= cov << 8;
+  const uint32_t paged = (uint32_t)(cov >> 15) & 0xFFFFu;  // tokens of the group that are part of a page
 
-  if (full) {
+  if (own != 0) {
+    const uint32_t off = __builtin_ctz(own);  // wave-uniform
+    const int32_t s0 = __builtin_amdgcn_readlane(sl, 15 + off);
+    if (off != 0) {
+#pragma unroll
+      for (int tk = 0; tk < 2; ++tk) {
+        const size_t o = (size_t)(t0 + off + p + 8 * tk) * rowstride + (size_t)h * D + c * DPL;
+#pragma unroll
+        for (int k = 0; k < KW; ++k) raw[tk][k] = *reinterpret_cast<const uint4 *>(src + o + 8 * k);
+      }
+    }
     float x[2][DPL];
 #pragma unroll
     for (int tk = 0; tk < 2; ++tk)
@@ -330,14 +360,15 @@ __global__ __launch_bounds__(kThreads) void write_int4_pages_kernel(
     if (c % GL == 0)
       __builtin_nontemporal_store(as_u32(half2_t{page_scale(sc[0]), page_scale(sc[1])}),
                                   reinterpret_cast<uint32_t *>(blk + scales_off + 2 * f.scale_idx(p, (c * DPL) / 64)));
-    return;
   }
+  if (paged == 0xFFFFu) return;
 
 #pragma unroll
   for (int u = 0; u < 16 * CPR / 64; ++u) {
     const uint32_t j = u * 64 + lane;
     const uint32_t t = t0 + j / CPR, cc = j % CPR;
-    if (t >= T) continue;  // a token's CPR (>= 8) chunks leave together: 64-groups stay whole
+    // a token's CPR (>= 8) chunks leave together: 64-groups stay whole
+    if (t >= T || ((paged >> (j / CPR)) & 1)) continue;
     float x[8];
     unpack_half8(*reinterpret_cast<const uint4 *>(src + (size_t)t * rowstride + (size_t)h * D + cc * 8), x);
     float sc;
