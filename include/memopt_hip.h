@@ -99,6 +99,13 @@ int memopt_allocate_block(int64_t *block_idx);
 /* Replaces free_block(block_idx) — src/csrc/kv_cache.cu:179-185. */
 int memopt_free_block(int64_t block_idx);
 
+/* `count` calls of memopt_allocate_block / memopt_free_block as one, in the
+ * same FIFO order (a prompt takes hundreds of pages at a time). All or none:
+ * allocate leaves the list as it is and sets block_idx[0] = -1 when fewer
+ * than `count` blocks are free; free checks every index first. */
+int memopt_allocate_blocks(int64_t count, int64_t *block_idx);
+int memopt_free_blocks(int64_t count, const int64_t *block_idx);
+
 /* Replaces free_blocks_count() — src/csrc/kv_cache.cu:198-201. */
 int memopt_free_blocks_count(int64_t *count);
 

@@ -155,6 +155,33 @@ int memopt_free_block(int64_t block_idx) {
   return MEMOPT_OK;
 }
 
+int memopt_allocate_blocks(int64_t count, int64_t *block_idx) {
+  std::lock_guard<std::mutex> lk(g_pool.mu);
+  MEMOPT_REQUIRE(g_pool.view.initialized, MEMOPT_ERR_STATE, "allocate_blocks: pool not initialized");
+  MEMOPT_REQUIRE(count >= 0 && (block_idx || count == 0), MEMOPT_ERR_INVALID, "allocate_blocks: bad arguments");
+  if (count == 0) return MEMOPT_OK;
+  if ((int64_t)g_pool.free_list.size() < count) {
+    block_idx[0] = -1;
+    return MEMOPT_OK;
+  }
+  for (int64_t i = 0; i < count; ++i) {
+    block_idx[i] = g_pool.free_list.front();
+    g_pool.free_list.pop_front();
+  }
+  return MEMOPT_OK;
+}
+
+int memopt_free_blocks(int64_t count, const int64_t *block_idx) {
+  std::lock_guard<std::mutex> lk(g_pool.mu);
+  MEMOPT_REQUIRE(g_pool.view.initialized, MEMOPT_ERR_STATE, "free_blocks: pool not initialized");
+  MEMOPT_REQUIRE(count >= 0 && (block_idx || count == 0), MEMOPT_ERR_INVALID, "free_blocks: bad arguments");
+  for (int64_t i = 0; i < count; ++i)
+    MEMOPT_REQUIRE(block_idx[i] >= 0 && block_idx[i] < g_pool.view.num_blocks, MEMOPT_ERR_INVALID,
+                   "free_blocks: block_idx out of range");
+  for (int64_t i = 0; i < count; ++i) g_pool.free_list.push_back(block_idx[i]);
+  return MEMOPT_OK;
+}
+
 int memopt_free_blocks_count(int64_t *count) {
   std::lock_guard<std::mutex> lk(g_pool.mu);
   *count = (int64_t)g_pool.free_list.size();

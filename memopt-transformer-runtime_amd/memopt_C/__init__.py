@@ -28,10 +28,11 @@ The library is loaded at import; a missing or unloadable library raises
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
-from typing import List, Optional, Tuple
+from typing import List, Optional, Sequence, Tuple
 
 import torch  # must precede the HIP library so both share one HIP runtime
 
@@ -91,6 +92,8 @@ _c_set_storage = _sig("memopt_pool_set_storage", [_i32, _vp, _vp])
 _c_pages_to_fp16 = _sig("memopt_int4_pages_to_fp16", [_vp, _i64, _i32, _i32, _vp, _vp, _vp])
 _c_alloc = _sig("memopt_allocate_block", [ctypes.POINTER(_i64)])
 _c_free = _sig("memopt_free_block", [_i64])
+_c_alloc_n = _sig("memopt_allocate_blocks", [_i64, ctypes.POINTER(_i64)])
+_c_free_n = _sig("memopt_free_blocks", [_i64, ctypes.POINTER(_i64)])
 _c_free_count = _sig("memopt_free_blocks_count", [ctypes.POINTER(_i64)])
 _c_write = _sig("memopt_write_cache", [_vp, _vp, _i64, _i32, _i32, _vp, _vp])
 _c_evict_cache = _sig("memopt_evict_cache", [_vp, _i64, _f32, _i32, _vp])
@@ -115,7 +118,15 @@ def _check(rc: int) -> None:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing to enter where it is current already."""
+    return _SAME_DEVICE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -226,6 +237,18 @@ def free_block(block_idx: int) -> None:
     _check(_c_free(int(block_idx)))
 
 
+def allocate_blocks(count: int) -> Optional[List[int]]:
+    """``count`` blocks popped as ``allocate_block`` would; ``None``, and none taken, when fewer are free."""
+    out = (_i64 * max(1, count))()
+    _check(_c_alloc_n(count, out))
+    return None if count and out[0] < 0 else out[:count]
+
+
+def free_blocks(blocks: Sequence[int]) -> None:
+    """Return blocks to the free list in order; every index is checked before the first is returned."""
+    _check(_c_free_n(len(blocks), (_i64 * max(1, len(blocks)))(*blocks)))
+
+
 def free_blocks_count() -> int:
     out = _i64()
     _check(_c_free_count(ctypes.byref(out)))
@@ -291,7 +314,7 @@ def dequantize_int4_pages(pages: Optional[torch.Tensor] = None) -> Tuple[torch.T
     nb, H = pages.shape[0], pages.shape[1]
     k = torch.empty((nb, 16, H, D), dtype=torch.float16, device=pages.device)
     v = torch.empty_like(k)
-    with torch.cuda.device(pages.device):
+    with _on(pages.device):
         _check(_c_pages_to_fp16(pages.data_ptr(), nb, H, D, k.data_ptr(), v.data_ptr(), _stream(pages)))
     return k, v
 
@@ -320,7 +343,7 @@ def convert_pool(kv_format: str) -> None:
             old_k, old_v = p["k"], p["v"]
             _check(_c_set_storage(KV_INT4, pages.data_ptr(), None))
             slots = torch.arange(nb * bs, dtype=torch.int32, device=dev)
-            with torch.cuda.device(dev):
+            with _on(dev):
                 _check(_c_write(old_k.data_ptr(), old_v.data_ptr(), nb * bs, H, D, slots.data_ptr(),
                                 _stream(old_k)))
             _pool.update(fmt=fmt, pages=pages, k=pages[:, :, lay["kcodes"]:lay["vcodes"]],
@@ -367,7 +390,7 @@ def write_cache(keys: torch.Tensor, values: torch.Tensor, block_tables: torch.Te
     if validate_slots:
         lo, hi = (int(x) for x in torch.aminmax(slot_mapping))
         _require(lo >= 0 and hi < p["nb"] * p["bs"], "write_cache: slot_mapping out of bounds")
-    with torch.cuda.device(keys.device):
+    with _on(keys.device):
         _check(_c_write(keys.data_ptr(), values.data_ptr(), T, H, D, slot_mapping.data_ptr(), _stream(keys)))
 
 
@@ -389,7 +412,7 @@ def evict_cache(block_tables: torch.Tensor, attention_scores: torch.Tensor, reta
     _require(h == p["h"], "evict_cache: attention_scores num_heads != pool.num_heads")
     _cuda(attention_scores, "attention_scores", "evict_cache")
     scores = attention_scores.contiguous()
-    with torch.cuda.device(scores.device):
+    with _on(scores.device):
         _check(_c_evict_cache(scores.data_ptr(), nb, float(retain_ratio), int(num_sink_tokens), _stream(scores)))
 
 
@@ -436,7 +459,7 @@ def evict_tokens(attention_scores: torch.Tensor, block_tables: torch.Tensor, is_
     scores = attention_scores.contiguous()
     M, nb = block_tables.shape[1], is_block_free.shape[0]
     need = evict_workspace_bytes(N, H, L, M, nb)
-    with torch.cuda.device(scores.device):
+    with _on(scores.device):
         if workspace is None:
             # scratch from torch's caching allocator on the current stream (page
             # marks and long-row selection state; nothing is kept between calls)
@@ -487,7 +510,7 @@ def quantize_kv_cache_int4(cache: torch.Tensor, group_size: int) -> List[torch.T
     packed = torch.empty(cache.shape[:-1] + (last // 2,), dtype=torch.uint8, device=cache.device)
     scales = torch.empty((n // group_size,), dtype=torch.float32, device=cache.device)
     if n:
-        with torch.cuda.device(cache.device):
+        with _on(cache.device):
             _check(_c_quant(cache.data_ptr(), n, last, group_size, packed.data_ptr(), scales.data_ptr(),
                             _stream(cache)))
     return [packed, scales]
@@ -507,7 +530,7 @@ def dequantize_kv_cache_int4(q_cache: torch.Tensor, scales: torch.Tensor, group_
              f"dequantize_kv_cache_int4: scales length ({scales.numel()}) != expected num_groups ({total // 64})")
     out = torch.empty(q_cache.shape[:-1] + (q_cache.shape[-1] * 2,), dtype=torch.float16, device=q_cache.device)
     if total:
-        with torch.cuda.device(q_cache.device):
+        with _on(q_cache.device):
             _check(_c_dequant(q_cache.data_ptr(), q_cache.numel(), scales.data_ptr(), scales.numel(), group_size,
                               out.data_ptr(), _stream(q_cache)))
     return out
@@ -554,25 +577,30 @@ def _attention_desc(query, key_cache, value_cache, block_tables, context_lens, m
 
     Returns (desc, out, workspace, keepalive) or (None, out, None, ()) for empty shapes.
     """
+    # (A message with values in it is formatted only when it is raised: on a
+    # small decode the host side of the call is longer than its kernels.)
     fn = "dynamic_sparse_attention"
     for t, n in ((query, "query"), (key_cache, "key_cache"), (value_cache, "value_cache"),
                  (block_tables, "block_tables"), (context_lens, "context_lens")):
-        _require(isinstance(t, torch.Tensor) and t.is_cuda, f"{n} must be a CUDA tensor")
+        if not (isinstance(t, torch.Tensor) and t.is_cuda):
+            raise RuntimeError(f"{n} must be a CUDA tensor")
     for t, n in ((query, "query"), (block_tables, "block_tables"), (context_lens, "context_lens")):
-        _require(t.is_contiguous(), f"{n} must be contiguous")
-    _require(query.dim() == 4, "query must be 4-D [batch, q_len, num_heads, head_dim]")
-    _require(block_tables.dim() == 2, "block_tables must be 2-D [batch, max_blocks_per_seq]")
-    _require(context_lens.dim() == 1, "context_lens must be 1-D [batch]")
+        if not t.is_contiguous():
+            raise RuntimeError(f"{n} must be contiguous")
+    q_shape, bt_shape, cl_shape = query.shape, block_tables.shape, context_lens.shape
+    _require(len(q_shape) == 4, "query must be 4-D [batch, q_len, num_heads, head_dim]")
+    _require(len(bt_shape) == 2, "block_tables must be 2-D [batch, max_blocks_per_seq]")
+    _require(len(cl_shape) == 1, "context_lens must be 1-D [batch]")
     _require(query.dtype == torch.float16, "query must be fp16")
     _require(block_tables.dtype == torch.int32, "block_tables must be int32")
     _require(context_lens.dtype == torch.int32, "context_lens must be int32")
-    B, Lq, H, D = query.shape
-    _require(block_tables.shape[0] == B, "block_tables batch dimension mismatch")
-    _require(context_lens.shape[0] == B, "context_lens batch dimension mismatch")
+    B, Lq, H, D = q_shape
+    _require(bt_shape[0] == B, "block_tables batch dimension mismatch")
+    _require(cl_shape[0] == B, "context_lens batch dimension mismatch")
     if out is None:
         out = torch.empty_like(query)
-    _require(out.shape == query.shape and out.dtype == torch.float16 and out.is_contiguous() and out.is_cuda,
-             f"{fn}: out must be a contiguous fp16 CUDA tensor shaped like query")
+    elif not (out.shape == q_shape and out.dtype == torch.float16 and out.is_contiguous() and out.is_cuda):
+        raise RuntimeError(f"{fn}: out must be a contiguous fp16 CUDA tensor shaped like query")
     keep = (query, key_cache, value_cache, block_tables, context_lens, key_scales, value_scales)
     fmt = KV_FP16
     sc = (0, 0, 0)
@@ -581,7 +609,7 @@ def _attention_desc(query, key_cache, value_cache, block_tables, context_lens, m
     base_k, base_v = key_cache.data_ptr(), value_cache.data_ptr()
     if key_cache.dtype == torch.uint8:
         _require(value_cache.dtype == torch.uint8, "value_cache must match key_cache (INT4 codes)")
-        _require(D % 64 == 0, f"{fn}: INT4 caches need head_dim % 64 == 0")
+        _require(D % 64 == 0, "dynamic_sparse_attention: INT4 caches need head_dim % 64 == 0")
         pages = _int4_pages_base(key_cache, value_cache, H, D) if kv_layout in (None, "pages") else None
         if pages is not None:
             fmt = KV_INT4
@@ -590,46 +618,43 @@ def _attention_desc(query, key_cache, value_cache, block_tables, context_lens, m
             bs = 16
             keep = keep + (buf,)
         else:
-            _require(kv_layout in (None, "token_major"), f"{fn}: not an INT4 page buffer")
+            _require(kv_layout in (None, "token_major"), "dynamic_sparse_attention: not an INT4 page buffer")
             _require(key_cache.dim() == 4 and value_cache.shape == key_cache.shape and value_cache.is_contiguous(),
                      "key_cache must be 4-D [num_kv_blocks, block_size, num_heads, head_dim/2] (INT4 codes)")
-            _require(key_scales is not None and value_scales is not None, f"{fn}: INT4 caches need key/value scales")
+            _require(key_scales is not None and value_scales is not None,
+                     "dynamic_sparse_attention: INT4 caches need key/value scales")
             for t, n in ((key_scales, "key_scales"), (value_scales, "value_scales")):
-                _require(t.is_cuda and t.is_contiguous(), f"{n} must be a contiguous CUDA tensor")
+                if not (t.is_cuda and t.is_contiguous()):
+                    raise RuntimeError(f"{n} must be a contiguous CUDA tensor")
             _require(key_scales.dtype == value_scales.dtype and key_scales.shape == value_scales.shape,
-                     f"{fn}: key/value scales mismatch")
+                     "dynamic_sparse_attention: key/value scales mismatch")
             fmt = KV_INT4_ROWS
             bs, nb, kv, sc, sdt = _int4_rows_layout(key_cache, key_scales, H, D)
     else:
         for t, n in ((key_cache, "key_cache"), (value_cache, "value_cache")):
-            _require(t.is_contiguous(), f"{n} must be contiguous")
-        _require(key_cache.dim() == 4, "key_cache must be 4-D [num_kv_blocks, block_size, num_heads, head_dim]")
-        _require(value_cache.dim() == 4, "value_cache must be 4-D [num_kv_blocks, block_size, num_heads, head_dim]")
+            if not t.is_contiguous():
+                raise RuntimeError(f"{n} must be contiguous")
+        k_shape, v_shape = key_cache.shape, value_cache.shape
+        _require(len(k_shape) == 4, "key_cache must be 4-D [num_kv_blocks, block_size, num_heads, head_dim]")
+        _require(len(v_shape) == 4, "value_cache must be 4-D [num_kv_blocks, block_size, num_heads, head_dim]")
         _require(key_cache.dtype == torch.float16, "key_cache must be fp16")
         _require(value_cache.dtype == torch.float16, "value_cache must be fp16")
-        nb, bs = key_cache.shape[0], key_cache.shape[1]
-        _require(key_cache.shape[2] == H, f"key_cache num_heads {key_cache.shape[2]} != query num_heads {H}")
-        _require(key_cache.shape[3] == D, f"key_cache head_dim {key_cache.shape[3]} != query head_dim {D}")
-        _require(value_cache.shape[1] == bs, "value_cache block_size mismatch")
-        _require(value_cache.shape[2] == H, "value_cache num_heads mismatch")
-        _require(value_cache.shape[3] == D, "value_cache head_dim mismatch")
+        nb, bs = k_shape[0], k_shape[1]
+        if k_shape[2] != H:
+            raise RuntimeError(f"key_cache num_heads {k_shape[2]} != query num_heads {H}")
+        if k_shape[3] != D:
+            raise RuntimeError(f"key_cache head_dim {k_shape[3]} != query head_dim {D}")
+        _require(v_shape[1] == bs, "value_cache block_size mismatch")
+        _require(v_shape[2] == H, "value_cache num_heads mismatch")
+        _require(v_shape[3] == D, "value_cache head_dim mismatch")
         kv = (bs * H * D, D, H * D)
     if B == 0 or Lq == 0 or H == 0 or D == 0:
         return None, out, None, ()
-    d = AttnDesc()
-    d.query, d.out = query.data_ptr(), out.data_ptr()
-    d.batch, d.q_len, d.num_heads, d.head_dim = B, Lq, H, D
-    d.kv_format = fmt
-    d.key_cache, d.value_cache = base_k, base_v
-    if fmt == KV_INT4_ROWS:
-        d.key_scales, d.value_scales = key_scales.data_ptr(), value_scales.data_ptr()
-    d.scale_dtype, d.block_size, d.num_kv_blocks = sdt, bs, nb
-    d.kv_page_stride, d.kv_head_stride, d.kv_token_stride = kv
-    d.sc_page_stride, d.sc_head_stride, d.sc_token_stride = sc
-    d.block_tables, d.max_blocks_per_seq = block_tables.data_ptr(), block_tables.shape[1]
-    d.context_lens = context_lens.data_ptr()
-    d.max_seq_len, d.window_size = int(max_seq_len), int(window_size)
-    d.num_sink_tokens, d.causal = int(num_sink_tokens), int(bool(causal))
+    rows = fmt == KV_INT4_ROWS
+    d = AttnDesc(query.data_ptr(), out.data_ptr(), B, Lq, H, D, fmt, base_k, base_v,
+                 key_scales.data_ptr() if rows else None, value_scales.data_ptr() if rows else None, sdt, bs, nb,
+                 *kv, *sc, block_tables.data_ptr(), bt_shape[1], context_lens.data_ptr(), int(max_seq_len),
+                 int(window_size), int(num_sink_tokens), int(bool(causal)))
     need = _i64()
     _check(_c_ws(ctypes.byref(d), ctypes.byref(need)))
     ws = None
@@ -661,7 +686,7 @@ def dynamic_sparse_attention(query: torch.Tensor, key_cache: torch.Tensor, value
     ``key_scales`` / ``value_scales`` (``kv_layout="token_major"``).
     """
     _require(isinstance(query, torch.Tensor) and query.is_cuda, "query must be a CUDA tensor")
-    with torch.cuda.device(query.device):
+    with _on(query.device):
         d, out, ws, _keep = _attention_desc(query, key_cache, value_cache, block_tables, context_lens,
                                             max_seq_len, window_size, num_sink_tokens, causal, key_scales,
                                             value_scales, kv_layout, None)
@@ -690,7 +715,7 @@ class PreparedAttention:
                  no_alloc=False):
         _require(isinstance(query, torch.Tensor) and query.is_cuda, "query must be a CUDA tensor")
         self.device = query.device
-        with torch.cuda.device(self.device):
+        with _on(self.device):
             self._d, self.out, self._ws, self._keep = _attention_desc(
                 query, key_cache, value_cache, block_tables, context_lens, max_seq_len, window_size,
                 num_sink_tokens, causal, key_scales, value_scales, kv_layout, out, alloc_workspace=not no_alloc)
@@ -704,6 +729,6 @@ class PreparedAttention:
 
     def __call__(self, stream: Optional[int] = None) -> torch.Tensor:
         if self._dp is not None:
-            s = stream if stream is not None else torch.cuda.current_stream(self.device).cuda_stream
+            s = stream if stream is not None else torch._C._cuda_getCurrentRawStream(self.device.index)
             _check(self._fn(self._dp, s))
         return self.out

@@ -13,7 +13,7 @@ side only does list bookkeeping and builds the small index tensors.
 """
 from __future__ import annotations
 
-from typing import Dict, Iterable, List, Optional, Sequence
+from typing import Dict, Iterable, List, NamedTuple, Optional, Sequence
 
 import numpy as np
 import torch
@@ -25,18 +25,39 @@ def slots_for(pages: Sequence[int], start: int, count: int, block_size: int) -> 
     """Flat pool slots (``page * block_size + offset``) of token positions
     ``start .. start + count - 1`` of a sequence whose logical blocks map to
     ``pages`` (the slot_mapping convention of src/csrc/kv_cache.cu:244-259)."""
-    out = []
-    for pos in range(start, start + count):
-        page = pages[pos // block_size]
-        if page < 0:
-            raise RuntimeError(f"slot of position {pos}: logical block {pos // block_size} is unlinked")
-        out.append(page * block_size + pos % block_size)
-    return out
+    return _slots_array(pages, start, count, block_size).tolist()
+
+
+def _slots_array(pages: Sequence[int], start: int, count: int, block_size: int) -> np.ndarray:
+    pos = np.arange(start, start + count)
+    page = np.asarray(pages, dtype=np.int64)[pos // block_size]
+    if count and page.min() < 0:
+        p = int(pos[page < 0][0])
+        raise RuntimeError(f"slot of position {p}: logical block {p // block_size} is unlinked")
+    return page * block_size + pos % block_size
+
+
+def upload_indices(values: np.ndarray, device: torch.device) -> torch.Tensor:
+    """int32 copy of ``values`` on ``device``, ordered on the current stream
+    and not waited for: from pinned memory, whose block torch's host allocator
+    keeps until the copy is done. (A copy from pageable memory waits for the
+    work queued before it, so the host could not run ahead of the GPU.) For
+    tensors that the current stream alone uses."""
+    host = torch.empty(values.shape, dtype=torch.int32, pin_memory=True)
+    host.numpy()[...] = values
+    return host.to(device, non_blocking=True)
 
 
 def pages_needed(length: int, block_size: int) -> int:
     """Logical blocks covering ``length`` tokens."""
     return (length + block_size - 1) // block_size
+
+
+class PromptIndices(NamedTuple):
+    """int32 views: slots ``[tokens]``, block table ``[1, pages]``, context lengths ``[calls]``."""
+    slots: torch.Tensor
+    table: torch.Tensor
+    lens: torch.Tensor
 
 
 class PagedKVCache:
@@ -90,9 +111,7 @@ class PagedKVCache:
 
     def free_sequence(self, seq_id: int) -> None:
         """Return the sequence's linked pages to the pool's free list."""
-        for page in self._pages.pop(seq_id):
-            if page >= 0:
-                memopt_C.free_block(page)
+        memopt_C.free_blocks([page for page in self._pages.pop(seq_id) if page >= 0])
         del self._len[seq_id]
 
     def length(self, seq_id: int) -> int:
@@ -103,18 +122,13 @@ class PagedKVCache:
 
     def reserve(self, seq_id: int, new_tokens: int) -> None:
         """Allocate the pages ``new_tokens`` more tokens need. On exhaustion
-        the pages taken by this call go back and ``RuntimeError`` is raised
+        none is taken and ``RuntimeError`` is raised
         (``allocate_block`` returns -1, src/csrc/kv_cache.cu:163-172)."""
         pages = self._pages[seq_id]
         need = pages_needed(self._len[seq_id] + new_tokens, self.block_size) - len(pages)
-        taken = []
-        for _ in range(max(0, need)):
-            b = memopt_C.allocate_block()
-            if b < 0:
-                for t in taken:
-                    memopt_C.free_block(t)
-                raise RuntimeError(f"PagedKVCache: pool exhausted (sequence {seq_id} needs {need} more pages)")
-            taken.append(b)
+        taken = memopt_C.allocate_blocks(max(0, need))
+        if taken is None:
+            raise RuntimeError(f"PagedKVCache: pool exhausted (sequence {seq_id} needs {need} more pages)")
         pages.extend(taken)
 
     # -- index tensors ------------------------------------------------------
@@ -135,10 +149,18 @@ class PagedKVCache:
 
     def slot_mapping(self, seq_ids: Sequence[int], new_tokens: int) -> torch.Tensor:
         """int32 slots of the next ``new_tokens`` positions of each sequence (sequence-major)."""
-        slots: List[int] = []
-        for s in seq_ids:
-            slots += slots_for(self._pages[s], self._len[s], new_tokens, self.block_size)
-        return torch.from_numpy(np.array(slots, dtype=np.int32)).to(self.device)
+        slots = [_slots_array(self._pages[s], self._len[s], new_tokens, self.block_size) for s in seq_ids]
+        return torch.from_numpy(np.concatenate(slots or [np.empty(0)]).astype(np.int32)).to(self.device)
+
+    def prompt_indices(self, seq_id: int, tokens: int, ends: Sequence[int]) -> "PromptIndices":
+        """Index tensors of the sequence's next ``tokens`` positions (reserved
+        already) for calls that end at context lengths ``ends``: one upload,
+        for use on the current stream."""
+        pages = self._pages[seq_id]
+        slots = _slots_array(pages, self._len[seq_id], tokens, self.block_size)
+        dev = upload_indices(np.concatenate([slots, pages, ends]), self.device)
+        m = tokens + len(pages)
+        return PromptIndices(dev[:tokens], dev[tokens:m].unsqueeze(0), dev[m:])
 
     # -- writes -------------------------------------------------------------
     def append(self, seq_ids: Sequence[int], keys: torch.Tensor, values: torch.Tensor) -> None:
@@ -156,13 +178,19 @@ class PagedKVCache:
             raise RuntimeError("append: keys batch != number of sequences")
         for s in seq_ids:
             self.reserve(s, T)
-        slots = self.slot_mapping(seq_ids, T)
-        bt = self.block_tables(seq_ids)
-        # Slots come from pages this cache allocated: in range by construction.
-        memopt_C.write_cache(keys.reshape(B * T, H, D), values.reshape(B * T, H, D), bt, slots,
-                             validate_slots=False)
+        slots = upload_indices(np.concatenate([_slots_array(self._pages[s], self._len[s], T, self.block_size)
+                                               for s in seq_ids] or [np.empty(0, np.int64)]), self.device)
+        self.write_rows(seq_ids, keys.reshape(B * T, H, D), values.reshape(B * T, H, D), slots)
+
+    def write_rows(self, seq_ids: Sequence[int], keys: torch.Tensor, values: torch.Tensor,
+                   slots: torch.Tensor) -> None:
+        """Write rows ``[B * T, H, D]`` to the slots of the next T positions of
+        every sequence and advance the lengths. The slots come from pages this
+        cache reserved, so they are in range; ``write_cache`` takes no part of
+        the block tables."""
+        memopt_C.write_cache(keys, values, None, slots, validate_slots=False)
         for s in seq_ids:
-            self._len[s] += T
+            self._len[s] += keys.shape[0] // len(seq_ids)
 
     # -- eviction -------------------------------------------------------------
     def evict(self, seq_ids: Sequence[int], scores: torch.Tensor, retain_ratio: float,
