@@ -184,15 +184,25 @@ __global__ __launch_bounds__(256, QB == 1 && (FMT == MEMOPT_KV_INT4 || D == 64) 
   };
   const int32_t *btrow = p.bt + (int64_t)b * p.M;
   const int32_t cpp = PAGES ? 1 : p.bs >> 4;
-  auto lookup = [&](int32_t i) __attribute__((always_inline)) {
+  const int32_t nb32 = (int32_t)min(p.nb, (int64_t)INT32_MAX);
+  struct Entry {  // a chunk's block-table entry, not yet waited for
+    int32_t lc, page, phys;
+    bool in;
+  };
+  auto fetch = [&](int32_t i) __attribute__((always_inline)) {
+    Entry e;
+    e.lc = i < sc ? i : wc0 + (i - sc);
+    e.in = i < n_vis;
+    e.page = cpp == 1 ? e.lc : e.lc / cpp;
+    e.phys = btrow[e.in ? e.page : 0];  // n_vis > 0 here, so the row has an entry 0
+    return e;
+  };
+  auto resolve = [&](const Entry &e) __attribute__((always_inline)) {
     Chunk c;
-    c.lc = i < sc ? i : wc0 + (i - sc);
-    const bool in = i < n_vis;
-    const int32_t page = cpp == 1 ? c.lc : c.lc / cpp;
-    const int32_t phys = btrow[in ? page : 0];  // n_vis > 0 here, so the row has an entry 0
-    c.ok = in && phys >= 0 && phys < p.nb;
-    const int64_t pg = c.ok ? phys : 0;
-    const int32_t pos = c.ok ? 16 * (c.lc - page * cpp) : 0;
+    c.lc = e.lc;
+    c.ok = e.in && e.phys >= 0 && e.phys < nb32;
+    const int64_t pg = c.ok ? e.phys : 0;
+    const int32_t pos = c.ok ? 16 * (e.lc - e.page * cpp) : 0;
     c.kv = pg * p.kv_ps + (int64_t)h * p.kv_hs + (int64_t)pos * p.kv_ts;
     c.sc = ROWS ? pg * p.sc_ps + (int64_t)h * p.sc_hs + (int64_t)pos * p.sc_ts : 0;
     return c;
@@ -367,13 +377,16 @@ __global__ __launch_bounds__(256, QB == 1 && (FMT == MEMOPT_KV_INT4 || D == 64) 
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = fmaf(s[qb][e & 1][e >> 1], p.qk_scale_log2, ncm[qb]);
       if (!full) {
+        // (bounds relative to the lane's first key, one test per element and
+        // no branch: as short-circuited conditions a masked step took about
+        // 1200 instructions more than a full one)
         const int32_t pos = ctx - p.Lq + q0 + 16 * qb + r;
+        const int32_t last = c_ok ? (causal ? min(pos, kv_lim - 1) : kv_lim - 1) - key0 : -1;
+        const int32_t first_w = (causal ? pos - p.W + 1 : ctx - p.W) - key0, end_s = p.sinks - key0;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int32_t key = key0 + (e >> 1) + 8 * (e & 1);
-          const bool vis = c_ok && key < kv_lim &&
-                           (causal ? key <= pos && (key < p.sinks || key >= pos - p.W + 1)
-                                   : key >= ctx - p.W || key < p.sinks);
+          const int32_t c = (e >> 1) + 8 * (e & 1);
+          const bool vis = (c <= last) & ((c >= first_w) | (c < end_s));
           x[e] = vis ? x[e] : -INFINITY;
         }
       }
@@ -419,13 +432,14 @@ __global__ __launch_bounds__(256, QB == 1 && (FMT == MEMOPT_KV_INT4 || D == 64) 
     // V of tokens past the context or without a page may hold any bits; it
     // becomes zero, as P = 0 must not meet NaN.
     if (!full) {
+      const int32_t live_c = c_ok ? kv_lim - key0 : 0;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const bool live = c_ok && key0 + (e >> 1) + 8 * (e & 1) < kv_lim;
+        const bool live = (e >> 1) + 8 * (e & 1) < live_c;
         if constexpr (PAGES) {
-          if (!live) vr.sc[e >> 1] &= (e & 1) ? 0x0000FFFFu : 0xFFFF0000u;
+          vr.sc[e >> 1] &= live ? ~0u : (e & 1) ? 0x0000FFFFu : 0xFFFF0000u;
         } else if constexpr (ROWS) {
-          if (!live) vr.sc[e] = 0.0f;
+          vr.sc[e] = live ? vr.sc[e] : 0.0f;
         } else {
 #pragma unroll
           for (int j = 0; j < D / 32; ++j) vr.w[e][j] = live ? vr.w[e][j] : 0u;
@@ -474,14 +488,15 @@ __global__ __launch_bounds__(256, QB == 1 && (FMT == MEMOPT_KV_INT4 || D == 64) 
 
   int32_t st = begin + wave;
   if (st < end) {
-    Chunk ca = lookup(2 * st), cb = lookup(2 * st + 1);
+    Entry ea = fetch(2 * (st + NW)), eb = fetch(2 * (st + NW) + 1);
+    Chunk ca = resolve(fetch(2 * st)), cb = resolve(fetch(2 * st + 1));
     load_k(ca, cb);
     load_v(ca, cb);
     for (; st < end; st += NW) {
-      const bool more = st + NW < end;
-      const int32_t nx = more ? st + NW : st;
-      const Chunk na = lookup(2 * nx), nb_ = lookup(2 * nx + 1);
-      step(ca, cb, na, nb_, more);
+      const Chunk na = resolve(ea), nb_ = resolve(eb);
+      ea = fetch(2 * (st + 2 * NW));
+      eb = fetch(2 * (st + 2 * NW) + 1);
+      step(ca, cb, na, nb_, st + NW < end);
       ca = na;
       cb = nb_;
     }
@@ -493,7 +508,7 @@ __global__ __launch_bounds__(256, QB == 1 && (FMT == MEMOPT_KV_INT4 || D == 64) 
       // dims, and adds its quarter of V (the row sums have the token already).
 #pragma unroll 1
       for (int32_t i = 2 * (begin + wave); i < 2 * end; i += (i & 1) ? 2 * NW - 1 : 1) {
-        const Chunk c = lookup(i);
+        const Chunk c = resolve(fetch(i));
 #pragma unroll 1
         for (int t = 0; t < 16 && c.ok; ++t) {
           const int32_t key = c.lc * 16 + t;
