@@ -60,6 +60,7 @@ struct DecodeParams {
   int32_t pages;                // 1: this build's INT4 page format (page_format.hpp)
   int32_t M, H, W, sinks, splits;
   int32_t bs;           // tokens per page (fp16 pools; a multiple of 16)
+  int32_t hc;           // heads per cluster (token-major codes; 1: grid order)
   float qk_scale_log2;  // (1/sqrt(D)) * log2(e)
   float *ws_o;          // [B, H, splits, D] (splits > 1)
   float *ws_ml;         // [B, H, splits, 2]

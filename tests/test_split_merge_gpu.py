@@ -74,3 +74,17 @@ def test_captured_split_decode_replays():
             graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(call.out, want)
+
+
+@pytest.mark.parametrize("B,H", [(1, 1), (1, 8), (2, 12), (3, 5), (8, 3), (16, 6), (1, 40)])
+def test_token_major_head_clusters(B, H):
+    """Head counts and batches whose clusters cover all heads, a fraction, or
+    none: every (sequence, head) is computed once, in its place."""
+    rng = np.random.default_rng(B * 100 + H)
+    ctx = [int(x) for x in rng.integers(1, 90, B)]
+    q, k, v, bt, cl = _case(B + H, B, H, 64, ctx)
+    (kq, ks), (vq, vs) = O.quantize_int4(k), O.quantize_int4(v)
+    want = O.paged_attention(q, O.dequantize_int4(kq, ks), O.dequantize_int4(vq, vs), bt, cl, 128, 128)
+    got = memopt_C.dynamic_sparse_attention(to_dev(q), to_dev(kq), to_dev(vq), to_dev(bt), to_dev(cl), 128, 128,
+                                            key_scales=to_dev(ks), value_scales=to_dev(vs), kv_layout="token_major")
+    assert_close(got, want, what=f"{B} x {H} token-major heads")
