@@ -635,20 +635,38 @@ __global__ __launch_bounds__(256) void direct_merge_kernel(const DirectParams p,
 static int direct_qb(const memopt_attn_desc &d) { return d.q_len <= 16 ? 1 : 2; }
 
 // Where the direct kernel beats the staged path (staging and attention
-// launches together, measured on both sides with 5 to 40 heads, batches of 1
-// to 16, contexts of 300 to 16384 tokens):
+// launches together, both sides measured with 8 to 40 heads, batches of 1 to
+// 16, contexts of 300 to 16384 tokens, over pages / fp16 pools):
 //  * up to 192 queries, whatever the batch: staging costs about what 128
-//    queries compute (16 sequences of 1024 tokens x 32 heads, 128 queries:
-//    86 us against 122 over pages, 161 against 173 over fp16; at 256 queries
-//    on 4 sequences of 2048 tokens 70 against 77, but 101 against 94);
-//  * calls whose 128-query tiles leave the staged path's grid small: up to
-//    128 tiles at D = 128 (32 heads, 512 queries over 2048 tokens: 51
-//    against 54 us, over 16384: 244 against 372; at 160 tiles 94 against 86)
-//    and 256 at D = 64 (8 heads, 2000 queries: 25 against 52; 80 heads, 512
-//    queries, 320 tiles: 52 against 54 over pages, 60 against 55 over fp16).
+//    queries compute (8 sequences of 2000 tokens x 32 heads, 128 queries: 67
+//    against 142 us / 146 against 177; 4 of 8192, 192 queries: 186 against
+//    302 / 335 against 374; 4 of 2048, 256 queries: 65 against 76 / 99
+//    against 94);
+//  * up to 128 tiles of 128 queries, which leave half of the CUs idle on the
+//    staged path (32 heads, 512 queries over 2048 tokens: 51 against 54 us
+//    over pages, over 16384: 244 against 372);
+//  * little work per call, where the staging launch and the ramp of the long
+//    tiles weigh more than the staged path's faster inner loop: by (query,
+//    key) pairs over all heads, up to 32 / 24 million at D = 128 (25 M, 8
+//    heads x 2500 queries: 44 against 74 us / 47 against 74; 34 M, 32 heads x
+//    1024 queries, window 1024: 44 against 46 / 51 against 47; 50 M: 64
+//    against 55 / 74 against 56) and 110 / 70 million at D = 64 (83 M, 12
+//    heads x 4413 queries, window 2048: 59 against 68 / 70 against 68; 154 M:
+//    101 against 88 / 121 against 94).
 static bool direct_faster(const memopt_attn_desc &d) {
-  const int64_t tiles = (int64_t)((d.q_len + 127) / 128) * d.num_heads * d.batch;
-  return d.q_len <= 192 || tiles <= (d.head_dim == 128 ? 128 : 256);
+  const int64_t q = d.q_len, tiles = (q + 127) / 128 * d.num_heads * d.batch;
+  if (q <= 192 || tiles <= 128) return true;
+  // Pairs of one sequence at the longest context the block table holds.
+  const int64_t T = (int64_t)d.max_blocks_per_seq * d.block_size;
+  const int64_t W = std::min<int64_t>(effective_window(d.window_size, d.max_seq_len), T);
+  int64_t pairs = q * W;
+  if (d.causal) {  // sum of min(W, pos + 1) over the query positions T - q .. T - 1
+    const int64_t lo = std::max<int64_t>(0, T - q), full = std::max(lo, std::min(W, T));
+    pairs = (full - lo) * (full + lo + 1) / 2 + (T - full) * W;
+  }
+  const bool pages = d.kv_format == MEMOPT_KV_INT4;
+  const int64_t most = d.head_dim == 128 ? (pages ? 32 : 24) : (pages ? 110 : 70);
+  return pairs * d.num_heads * d.batch <= most * 1000000;
 }
 
 bool direct_supported(const memopt_attn_desc &d) {
