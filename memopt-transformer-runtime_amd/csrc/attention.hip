@@ -195,7 +195,8 @@ static int validate(const memopt_attn_desc &d) {
 
 static int decode_workspace(const memopt_attn_desc &d, int32_t *splits, int64_t *bytes) {
   // Splits are sized in the kernels' 16-token units.
-  *splits = decode_splits(d.batch, d.num_heads, max_pages_visited(d) * (d.block_size / 16));
+  *splits = decode_splits(d.batch, d.num_heads, max_pages_visited(d) * (d.block_size / 16),
+                          d.kv_format != MEMOPT_KV_FP16);
   *bytes = decode_workspace_bytes(d.batch, d.num_heads, *splits, d.head_dim);
   return MEMOPT_OK;
 }

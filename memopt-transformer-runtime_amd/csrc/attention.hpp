@@ -186,8 +186,8 @@ __device__ __forceinline__ void decode_epilogue(const DecodeParams &p, int64_t b
   p.out[bh * D + d] = (half_t)(lt > 0.0f ? o / lt : 0.0f);
 }
 
-// Split count used by the INT4 decode kernel for this launch shape.
-int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited);
+// Split count used by the decode kernels for this launch shape.
+int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool int4);
 // Launches the split-K INT4 decode kernel (splits merged in-kernel).
 int launch_decode_int4(const DecodeParams &p, int32_t batch, int32_t D, int32_t scale_dtype,
                        hipStream_t stream);

@@ -555,18 +555,28 @@ static DecodeShape decode_shape() {
   return s;
 }
 
-int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited) {
+// Splits of a decode over `units` (b, h) pairs, measured for both formats
+// over 32 to 384 units and 1500 to 16000 tokens (MI355X, 256 CUs):
+//  * fewer units than CUs: as many splits as keep the grid within two
+//    workgroups per CU (INT4) or one (fp16, whose loads fill a CU's share
+//    alone). A grid past that runs in uneven rounds: 120 units of 6000 tokens,
+//    INT4 in 7, 4, 2 splits 24.9, 20.8, 21.6 us; fp16 70.9, 65.0, 63.7; 200
+//    units INT4 in 4, 2 splits 37.0, 31.5, fp16 in 4, 1 118.6, 106.0;
+//  * 256 to 511 units: 2 (unsplit is up to 8 % faster on equal lengths, but
+//    10 % slower on lengths from a third to the whole of 4000 tokens);
+//  * at least 4 page batches per wave, and INT4 contexts of up to 64 pages are
+//    not split: the merge and the cleared workspace cost more than the pages
+//    they save (64 pages, 8 heads of 64: 6.5 us unsplit, 8.3 in 2; 94 pages,
+//    32 heads of 128: 10.7 against 9.2 and 2 for the clearing).
+int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool int4) {
   const int64_t units = (int64_t)batch * heads;
   if (units <= 0) return 1;
   const DecodeShape sh = decode_shape();
-  // About 2 workgroups per CU; 3 when the batch has fewer (b, h) units than
-  // CUs (config 5's 128 units: 6 splits measured 1.5 % faster than 4, and
-  // 2, 3 or 8 slower).
-  const int64_t target_wgs = (units < compute_units() ? 3LL : 2LL) * compute_units();
-  int64_t s = (target_wgs + units - 1) / units;
-  // Keep at least 4 page batches per wave.
+  const int64_t cus = compute_units();
+  int64_t s = units < cus ? (int4 ? 2 : 1) * cus / units : (2 * cus + units - 1) / units;
   const int64_t cap = max_pages_visited / (4LL * sh.nw * sh.u);
   if (s > cap) s = cap;
+  if (int4 && max_pages_visited <= 64) s = 1;
   if (s < 1) s = 1;
   if (s > 64) s = 64;
   if (const char *e = std::getenv("MEMOPT_DECODE_SPLITS")) {
