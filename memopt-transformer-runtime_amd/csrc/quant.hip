@@ -43,12 +43,14 @@ __device__ __forceinline__ void load8(const half_t *p, float f[8]) {
 }
 
 // One lane = 8 consecutive elements; chunk i covers elements [8i, 8i+8).
-// VEC: four chunks per thread, i0 + r * stride, all four non-temporal loads
-// issued before any is used (indices past the end load the last chunk and
-// store nothing; a group's 8 chunks are all in range or all out, as n_chunks
-// is a multiple of 8). With one chunk per thread, a launch of config 2's
-// pool tensor had four times the workgroups and ran at 0.72 of HBM, with
-// four 0.77 (eight 0.67).
+// VEC: four chunks per thread, i0 + r * kThreads, so a workgroup covers 16 KB
+// in one piece, all four non-temporal loads issued before any is used (indices
+// past the end load the last chunk and store nothing; a group's 8 chunks are
+// all in range or all out, as n_chunks is a multiple of 8). With the four
+// chunks a whole grid apart, each launch read four streams at once: 2039
+// pages of 16 x 32 x 128 quantized and restored took 109 us, 104 in one piece
+// (two chunks per thread 105, eight 111, plain loads 116, non-temporal code
+// stores 117); one chunk per thread ran at 0.72 of HBM where four reach 0.77.
 static constexpr int kQuantChunks = 4;
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void quantize_kernel(const half_t *__restrict__ in,
@@ -59,16 +61,16 @@ __global__ __launch_bounds__(kThreads) void quantize_kernel(const half_t *__rest
   if constexpr (VEC) {
     constexpr int R = kQuantChunks;
     typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-    for (int64_t i0 = (int64_t)blockIdx.x * kThreads + threadIdx.x; i0 < n_chunks; i0 += R * stride) {
+    for (int64_t i0 = (int64_t)blockIdx.x * kThreads * R + threadIdx.x; i0 < n_chunks; i0 += R * stride) {
       u4v x[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int64_t i = min(i0 + r * stride, n_chunks - 1);
+        const int64_t i = min(i0 + r * kThreads, n_chunks - 1);
         x[r] = __builtin_nontemporal_load(reinterpret_cast<const u4v *>(in + i * 8));
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int64_t i = i0 + r * stride;
+        const int64_t i = i0 + r * kThreads;
         float v[8];
         unpack_half8(make_uint4(x[r].x, x[r].y, x[r].z, x[r].w), v);
         float s;
@@ -106,21 +108,22 @@ __global__ __launch_bounds__(kThreads) void dequantize_kernel(const uint8_t *__r
                       as_u32(half2_t{h[6], h[7]}));
   };
   if constexpr (VEC) {
-    // Four chunks per trip, all loads issued before any is used: one 4-byte
-    // load per trip left too few bytes in flight to cover HBM latency.
+    // Four chunks per trip, in one piece per workgroup, all loads issued before
+    // any is used: one 4-byte load per trip left too few bytes in flight to
+    // cover HBM latency.
     constexpr int R = 4;
-    for (int64_t i0 = (int64_t)blockIdx.x * kThreads + threadIdx.x; i0 < n_chunks; i0 += R * stride) {
+    for (int64_t i0 = (int64_t)blockIdx.x * kThreads * R + threadIdx.x; i0 < n_chunks; i0 += R * stride) {
       uint32_t w[R];
       float sc[R];
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int64_t i = min(i0 + r * stride, n_chunks - 1);
+        const int64_t i = min(i0 + r * kThreads, n_chunks - 1);
         w[r] = reinterpret_cast<const uint32_t *>(packed)[i];
         sc[r] = scales[i >> 3];
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int64_t i = i0 + r * stride;
+        const int64_t i = i0 + r * kThreads;
         if (i < n_chunks) {
           const uint4 o = expand(w[r], sc[r]);
           typedef uint32_t u4v __attribute__((ext_vector_type(4)));
