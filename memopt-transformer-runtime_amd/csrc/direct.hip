@@ -652,7 +652,14 @@ static int direct_qb(const memopt_attn_desc &d) { return d.q_len <= 16 ? 1 : 2; 
 //    1024 queries, window 1024: 44 against 46 / 51 against 47; 50 M: 64
 //    against 55 / 74 against 56) and 110 / 70 million at D = 64 (83 M, 12
 //    heads x 4413 queries, window 2048: 59 against 68 / 70 against 68; 154 M:
-//    101 against 88 / 121 against 94).
+//    101 against 88 / 121 against 94);
+//  * few heads over long contexts: with at most two of its workgroups per CU
+//    the staged path takes as long as its longest tile, about 1.4 us per 64
+//    keys and 10 us, whatever the rest of the grid does, and the direct
+//    kernel 8 us and the pairs at its rate (8 heads of 128, 4000 causal
+//    queries: 83 against 106 us / 96 against 105, of 64: 55 against 91 / 62
+//    against 92; 8 of 64, 6000 queries, window 4096: 87 against 109 / 103
+//    against 110; 8 of 128, 8000 queries, window 2048: 123 against 86).
 static bool direct_faster(const memopt_attn_desc &d) {
   const int64_t q = d.q_len, tiles = (q + 127) / 128 * d.num_heads * d.batch;
   if (q <= 192 || tiles <= 128) return true;
@@ -665,8 +672,12 @@ static bool direct_faster(const memopt_attn_desc &d) {
     pairs = (full - lo) * (full + lo + 1) / 2 + (T - full) * W;
   }
   const bool pages = d.kv_format == MEMOPT_KV_INT4;
-  const int64_t most = d.head_dim == 128 ? (pages ? 32 : 24) : (pages ? 110 : 70);
-  return pairs * d.num_heads * d.batch <= most * 1000000;
+  const bool d128 = d.head_dim == 128;
+  const double mpairs = 1e-6 * (double)pairs * d.num_heads * d.batch;
+  if (mpairs <= (d128 ? (pages ? 32.0 : 24.0) : (pages ? 110.0 : 70.0))) return true;
+  const double rate = d128 ? (pages ? 0.85 : 0.68) : (pages ? 1.65 : 1.38);  // million pairs per us
+  const double keys = (double)std::min(T, d.causal ? W + 127 : W);           // of the longest tile
+  return tiles <= 2 * compute_units() && 8.0 + mpairs / rate < 0.9 * (10.0 + 1.4 * keys / 64);
 }
 
 bool direct_supported(const memopt_attn_desc &d) {
@@ -740,7 +751,7 @@ int launch_direct(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hip
   p.bt = d.block_tables;
   p.M = d.max_blocks_per_seq;
   p.ctx = d.context_lens;
-  p.W = W;
+  p.W = std::min(W, 1 << 30);  // (so that position - W stays in 32 bits for positions below 0)
   p.sinks = d.num_sink_tokens < 0 ? 0 : d.num_sink_tokens;
   p.causal = d.causal;
   p.qk_scale_log2 = qk_scale_log2;
