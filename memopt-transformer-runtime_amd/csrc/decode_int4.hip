@@ -558,10 +558,13 @@ static DecodeShape decode_shape() {
 // Splits of a decode over `units` (b, h) pairs, measured for both formats
 // over 32 to 384 units and 1500 to 16000 tokens (MI355X, 256 CUs):
 //  * fewer units than CUs: as many splits as keep the grid within two
-//    workgroups per CU (INT4) or one (fp16, whose loads fill a CU's share
-//    alone). A grid past that runs in uneven rounds: 120 units of 6000 tokens,
-//    INT4 in 7, 4, 2 splits 24.9, 20.8, 21.6 us; fp16 70.9, 65.0, 63.7; 200
-//    units INT4 in 4, 2 splits 37.0, 31.5, fp16 in 4, 1 118.6, 106.0;
+//    workgroups per CU; fp16, whose loads fill a CU's share alone, within one
+//    up to a quarter of the CUs, and 3 splits above half of them. A grid past
+//    that runs in uneven rounds: 120 units of 6000 tokens, INT4 in 7, 4
+//    splits 24.9, 20.8 us, fp16 70.9, 65.0; 64 units fp16 in 12, 4 40.8, 34.7;
+//    200 units INT4 in 4, 2 37.0, 31.5, fp16 in 4, 3 118.6, 107.9. Fewer lose
+//    on unequal lengths (160 units of 2000 to 5000 tokens, fp16 in 5, 3, 1
+//    splits 54.6, 53.9, 75.8);
 //  * 256 to 511 units: 2 (unsplit is up to 8 % faster on equal lengths, but
 //    10 % slower on lengths from a third to the whole of 4000 tokens);
 //  * at least 4 page batches per wave, and INT4 contexts of up to 64 pages are
@@ -573,7 +576,8 @@ int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool 
   if (units <= 0) return 1;
   const DecodeShape sh = decode_shape();
   const int64_t cus = compute_units();
-  int64_t s = units < cus ? (int4 ? 2 : 1) * cus / units : (2 * cus + units - 1) / units;
+  int64_t s = units < cus ? 2 * cus / units : (2 * cus + units - 1) / units;
+  if (!int4 && units < cus) s = 4 * units <= cus ? cus / units : 2 * units <= cus ? s : 3;
   const int64_t cap = max_pages_visited / (4LL * sh.nw * sh.u);
   if (s > cap) s = cap;
   if (int4 && max_pages_visited <= 64) s = 1;
