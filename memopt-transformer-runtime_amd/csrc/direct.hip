@@ -68,6 +68,17 @@ struct DirectParams {
   float *ws_o, *ws_ml;        // [B * H * Lq][splits][D], [B * H * Lq][splits][2]
 };
 
+// Output element from a query's weighted sum x and row sum l; 0 where no key
+// was visible. Where a score is NaN or +inf (an inf or NaN key scale, a query
+// that is not finite) l is NaN: over token-major codes the output is 0 then,
+// as the generic kernel's and the oracle's; over pages and fp16 pools x is NaN
+// and stays it, as on the staged path.
+template <bool ROWS>
+__device__ __forceinline__ half_t normalized(float x, float l) {
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  return ROWS && !(l > 0.0f) ? (half_t)0.0f : (half_t)(x * inv);
+}
+
 // Raw registers of one step, by cache format.
 template <int D, int FMT>
 struct DirectK;
@@ -577,8 +588,8 @@ __global__ __launch_bounds__(256, QB == 1 && (FMT == MEMOPT_KV_INT4 || D == 64) 
     }
     const int64_t qrow = ((int64_t)b * p.H + h) * p.Lq + qi;
     if (p.splits == 1) {
-      const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-      const half2_t y0 = {(half_t)(x[0] * inv), (half_t)(x[1] * inv)}, y1 = {(half_t)(x[2] * inv), (half_t)(x[3] * inv)};
+      const half2_t y0 = {normalized<ROWS>(x[0], l), normalized<ROWS>(x[1], l)};
+      const half2_t y1 = {normalized<ROWS>(x[2], l), normalized<ROWS>(x[3], l)};
       *reinterpret_cast<u32x2d_t *>(p.out + (((int64_t)b * p.Lq + qi) * p.H + h) * D + d) =
           u32x2d_t{as_u32(y0), as_u32(y1)};
     } else {
@@ -595,7 +606,7 @@ __global__ __launch_bounds__(256, QB == 1 && (FMT == MEMOPT_KV_INT4 || D == 64) 
 // Sums the splits of one query row, one wave per row: lane s takes split s's
 // (m, l) (splits <= 64); every lane then adds D / 64 dims over the splits,
 // eight loads in flight.
-template <int D>
+template <int D, bool ROWS>
 __global__ __launch_bounds__(256) void direct_merge_kernel(const DirectParams p, int64_t rows) {
   constexpr int R = 8, E = D / 64;
   typedef float vec_t __attribute__((ext_vector_type(E)));
@@ -622,12 +633,11 @@ __global__ __launch_bounds__(256) void direct_merge_kernel(const DirectParams p,
       if (s0 + k < p.splits) o += x[k] * fs;
     }
   }
-  const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
   const int32_t qi = (int32_t)(row % p.Lq);
   const int64_t bh = row / p.Lq, h = bh % p.H, b = bh / p.H;
   half_t *dst = p.out + ((b * p.Lq + qi) * p.H + h) * D + E * lane;
-  if constexpr (E == 2) *reinterpret_cast<uint32_t *>(dst) = as_u32(half2_t{(half_t)(o[0] * inv), (half_t)(o[1] * inv)});
-  else *dst = (half_t)(o[0] * inv);
+  if constexpr (E == 2) *reinterpret_cast<uint32_t *>(dst) = as_u32(half2_t{normalized<ROWS>(o[0], lt), normalized<ROWS>(o[1], lt)});
+  else *dst = normalized<ROWS>(o[0], lt);
 }
 
 // Query blocks of 16 * QB rows: two blocks of 16 share every K and V operand
@@ -777,8 +787,14 @@ int launch_direct(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hip
   int rc = check_launch("paged_attention(direct)");
   if (rc != MEMOPT_OK || p.splits == 1) return rc;
   const dim3 mgrid((unsigned)((rows + 3) / 4));
-  if (d.head_dim == 128) hipLaunchKernelGGL(direct_merge_kernel<128>, mgrid, dim3(256), 0, stream, p, rows);
-  else hipLaunchKernelGGL(direct_merge_kernel<64>, mgrid, dim3(256), 0, stream, p, rows);
+  const bool token_major = d.kv_format == MEMOPT_KV_INT4_ROWS;
+  if (d.head_dim == 128) {
+    if (token_major) hipLaunchKernelGGL((direct_merge_kernel<128, true>), mgrid, dim3(256), 0, stream, p, rows);
+    else hipLaunchKernelGGL((direct_merge_kernel<128, false>), mgrid, dim3(256), 0, stream, p, rows);
+  } else {
+    if (token_major) hipLaunchKernelGGL((direct_merge_kernel<64, true>), mgrid, dim3(256), 0, stream, p, rows);
+    else hipLaunchKernelGGL((direct_merge_kernel<64, false>), mgrid, dim3(256), 0, stream, p, rows);
+  }
   return check_launch("paged_attention(direct merge)");
 }
 
