@@ -109,3 +109,35 @@ def test_direct_rows_non_finite_values(D, scale):
                 assert ok.all() == (pos < key or h == 0)
                 assert_close(got[0, i, h][ok], want[ok], what=f"query {i} head {h}")
                 np.testing.assert_array_equal(got[0, i, h][~ok], want[~ok])
+
+
+@pytest.mark.parametrize("n", [200, 3000])                 # unsplit, and in splits
+@pytest.mark.parametrize("D,scale", [(64, np.nan), (128, np.nan), (64, np.inf)])
+def test_direct_rows_non_finite_scores(D, scale, n):
+    """Token-major codes with a NaN or inf K scale (codes of both signs in the
+    group, so the score is NaN), and a query holding a NaN: a query with such a
+    score gives zeros, as the oracle states; all others are as without it."""
+    B, H, bs, Lq, W, bad_q = 1, 2, 16, 40, 1 << 20, 3
+    q, k, v, bt, cl = _inputs(5, B, H, D, bs, [n], Lq, False)
+    (kq, ks), (vq, vs) = O.quantize_int4(k), O.quantize_int4(v)
+    key = n - 25                                     # seen by the last 25 queries, head 1
+    ks = ks.copy().reshape(-1, bs, H, D // 64)
+    ks[int(bt[0, key // bs]), key % bs, 1, 0] = scale
+    ks = ks.reshape(-1)
+    q[0, bad_q, 0, 7] = np.nan
+    args = (to_dev(q), to_dev(kq), to_dev(vq), to_dev(bt), to_dev(cl), n, W)
+    kw = dict(causal=True, key_scales=to_dev(ks), value_scales=to_dev(vs), kv_layout="token_major")
+    call = memopt_C.PreparedAttention(*args, **kw)
+    assert (call.workspace_bytes > 0) == (n == 3000)
+    got = call().cpu().numpy()
+    with np.errstate(all="ignore"):
+        want = O.paged_attention(q, O.dequantize_int4(kq, ks), O.dequantize_int4(vq, vs), bt, cl, n, W, causal=True)
+    # (the oracle's additive mask lets the NaN key reach queries before it; they are as with a finite one)
+    clean = O.paged_attention(q, O.dequantize_int4(kq, np.where(np.isfinite(ks), ks, 1).astype(ks.dtype)),
+                              O.dequantize_int4(vq, vs), bt, cl, n, W, causal=True)
+    hit = np.zeros((Lq, H), bool)
+    hit[Lq - 25:, 1] = True
+    hit[bad_q, 0] = True
+    assert (got[0][hit] == 0).all() and (want[0][hit] == 0).all()
+    assert_close(got[0][~hit], clean[0][~hit], what=f"queries without the score, n {n}")
+    assert_close(memopt_C.PreparedAttention(*args, no_alloc=True, **kw)(), got, what="no_alloc")
