@@ -690,7 +690,13 @@ static bool direct_faster(const memopt_attn_desc &d) {
   return tiles <= 2 * compute_units() && 8.0 + mpairs / rate < 0.9 * (10.0 + 1.4 * keys / 64);
 }
 
+static int64_t direct_query_blocks(const memopt_attn_desc &d) {
+  const int64_t qn = 16 * direct_qb(d);
+  return (d.q_len + qn - 1) / qn;
+}
+
 bool direct_supported(const memopt_attn_desc &d) {
+  if (direct_query_blocks(d) > 65535) return false;  // a grid dimension
   auto al = [](const void *x, int64_t a) { return ((uintptr_t)x & (uintptr_t)(a - 1)) == 0; };
   if (d.q_len < 2 || (d.head_dim != 64 && d.head_dim != 128) || d.num_kv_blocks <= 0) return false;
   if (!al(d.query, 16) || !al(d.out, 16)) return false;
@@ -709,7 +715,7 @@ bool direct_supported(const memopt_attn_desc &d) {
 static int32_t direct_splits(const memopt_attn_desc &d, int64_t bytes) {
   const int64_t rows = (int64_t)d.batch * d.num_heads * d.q_len;
   const int64_t qn = 16 * direct_qb(d);
-  const int64_t wgs = (int64_t)d.batch * d.num_heads * ((d.q_len + qn - 1) / qn);
+  const int64_t wgs = (int64_t)d.batch * d.num_heads * direct_query_blocks(d);
   const int64_t W = effective_window(d.window_size, d.max_seq_len);
   const int64_t sinks = d.num_sink_tokens > 0 ? d.num_sink_tokens : 0;
   int64_t tokens = (d.causal ? W + qn : W) + sinks + 32;
@@ -772,9 +778,9 @@ int launch_direct(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hip
     p.ws_ml = p.ws_o + rows * p.splits * d.head_dim;
   }
   const int qb = direct_qb(d);
-  const int64_t gx = (int64_t)d.batch * d.num_heads * p.splits, gy = (d.q_len + 16 * qb - 1) / (16 * qb);
-  MEMOPT_REQUIRE(gx < (1LL << 31) && gy <= 65535, MEMOPT_ERR_UNSUPPORTED, "paged_attention: too many query blocks");
-  const dim3 grid((unsigned)gx, (unsigned)gy);
+  const int64_t gx = (int64_t)d.batch * d.num_heads * p.splits;
+  MEMOPT_REQUIRE(gx < (1LL << 31), MEMOPT_ERR_UNSUPPORTED, "paged_attention: too many query blocks");
+  const dim3 grid((unsigned)gx, (unsigned)direct_query_blocks(d));
   if (d.head_dim == 128) {
     if (d.kv_format == MEMOPT_KV_INT4) launch_direct_qb<128, MEMOPT_KV_INT4>(p, qb, grid, stream);
     else if (d.kv_format == MEMOPT_KV_FP16) launch_direct_qb<128, MEMOPT_KV_FP16>(p, qb, grid, stream);

@@ -141,3 +141,17 @@ def test_direct_rows_non_finite_scores(D, scale, n):
     assert (got[0][hit] == 0).all() and (want[0][hit] == 0).all()
     assert_close(got[0][~hit], clean[0][~hit], what=f"queries without the score, n {n}")
     assert_close(memopt_C.PreparedAttention(*args, no_alloc=True, **kw)(), got, what="no_alloc")
+
+
+def test_more_query_blocks_than_a_grid_dimension():
+    """2097152 queries (65536 blocks of 32, one more than the direct kernel's
+    grid takes) with little work per query: served, as any other length."""
+    B, H, D, n, Lq, W = 1, 1, 64, 40, 65536 * 32, 16
+    q, k, v, bt, cl = _inputs(6, B, H, D, 16, [n], 2, False)
+    rows = torch.randn(4096, D, generator=torch.Generator().manual_seed(6)).half()
+    qd = rows.to(dev()).repeat(Lq // 4096, 1).reshape(B, Lq, H, D)
+    got = memopt_C.dynamic_sparse_attention(qd, to_dev(k), to_dev(v), to_dev(bt), to_dev(cl), n, W)
+    want = O.paged_attention(rows.numpy().reshape(1, 4096, 1, D), k, v, bt, cl, n, W)
+    assert_close(got[:, :4096], want, what="first queries")
+    same = got.reshape(Lq // 4096, 4096, D)
+    assert all(torch.equal(same[i], same[0]) for i in range(0, Lq // 4096, 37)) and torch.equal(same[-1], same[0])
