@@ -19,6 +19,7 @@
 //     online softmax. INT4 elements are dequantized to fp16 exactly as the
 //     reference's dequantize kernel would (fp16(RNE((code-8)*scale))) before
 //     use, so it computes the reference composition.
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -276,10 +277,12 @@ int memopt_attention_workspace_size(const memopt_attn_desc *desc, int64_t *bytes
     return decode_workspace(*desc, &splits, bytes);
   }
   // (INT4 pages and fp16 pools: the staged path's size, also where the direct
-  // kernel, which needs less, takes the call)
+  // kernel takes the call, whose partials are no larger; but the partials'
+  // where the staged copy would pass its 31 bits: 5 queries on 131072 tokens
+  // x 32 heads of 128 take 127 us in their 16 splits, 1218 in one)
   if (desc->batch > 0 && desc->num_heads > 0) {
     if (prefill_supported(*desc)) *bytes = prefill_workspace_bytes(*desc);
-    else if (direct_supported(*desc)) *bytes = direct_workspace_bytes(*desc);
+    if (direct_supported(*desc)) *bytes = std::max(*bytes, direct_workspace_bytes(*desc));
   }
   return MEMOPT_OK;
 }

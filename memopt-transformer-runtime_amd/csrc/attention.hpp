@@ -200,6 +200,7 @@ int launch_decode_fp16(const DecodeParams &p, int32_t batch, int32_t D, hipStrea
 bool prefill_supported(const memopt_attn_desc &d);
 // Workspace of the staged prefill path (0: the path stages in-kernel).
 int64_t prefill_workspace_bytes(const memopt_attn_desc &d);
+int64_t staged_copy_bytes(const memopt_attn_desc &d);  // the same, also past the sizes the staged path takes
 int launch_prefill(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hipStream_t stream);
 
 // Multi-query kernel without staging (direct.hip): calls over INT4 pages and

@@ -711,8 +711,16 @@ bool direct_supported(const memopt_attn_desc &d) {
 // Splits of a call: about two workgroups per CU (three or more: 12 % slower at
 // 16 sequences of 2000 fp16 tokens, 30 % at 64 queries of one sequence), at least two steps (64
 // tokens) per wave, at most 64, and no more than `bytes` of partials hold
-// (none without a workspace).
+// (none without a workspace). Over INT4 pages and fp16 pools the partials are
+// also no larger than the staged path's copy of K and V: with about as many
+// queries as keys, writing and merging them costs more than the idle CUs
+// (causal, 8 heads of 128, 1024 queries on 1024 tokens 17 us unsplit, 23 in 2
+// splits; 800 on 800 over fp16 15 and 24 in 3; 12 heads of 64, 512 on 512 9
+// and 13; with one or two heads they break even: 1100 on 1100 17 and 13 in 4,
+// 2 x 2000 on 2000 26 and 25). Both entry points and the workspace query
+// count by this rule, so they run the same splits wherever these fit.
 static int32_t direct_splits(const memopt_attn_desc &d, int64_t bytes) {
+  if (d.kv_format != MEMOPT_KV_INT4_ROWS) bytes = std::min(bytes, staged_copy_bytes(d));
   const int64_t rows = (int64_t)d.batch * d.num_heads * d.q_len;
   const int64_t qn = 16 * direct_qb(d);
   const int64_t wgs = (int64_t)d.batch * d.num_heads * direct_query_blocks(d);

@@ -1538,12 +1538,16 @@ static int64_t stage_counters_offset(const memopt_attn_desc &d, int64_t mc) {
   return (units * (64LL * d.head_dim) + (int64_t)d.batch * mc * 4 + 7) / 8 * 8;
 }
 
+int64_t staged_copy_bytes(const memopt_attn_desc &d) {
+  return stage_counters_offset(d, staged_chunks(d)) + (int64_t)d.batch * d.num_heads * 64 * 4;
+}
+
 int64_t prefill_workspace_bytes(const memopt_attn_desc &d) {
   const int64_t mc = staged_chunks(d);
   const int64_t units = (int64_t)d.batch * mc * d.num_heads;
   // one sequence's chunks must stay inside a 31-bit buffer range
   if (units <= 0 || units >= (1LL << 31) || mc * d.num_heads * 64LL * d.head_dim >= (1LL << 31)) return 0;
-  return stage_counters_offset(d, mc) + (int64_t)d.batch * d.num_heads * 64 * 4;
+  return staged_copy_bytes(d);
 }
 
 // Id of a prefill call for the in-kernel staging flags: 1 .. 2^32 - 1.

@@ -161,3 +161,29 @@ def test_paged_attention_requires_its_workspace(lib):
     attn.argtypes = [ctypes.POINTER(memopt_C.AttnDesc), ctypes.c_void_p]
     assert attn(ctypes.byref(d), None) == ERR_INVALID
     assert b"workspace too small" in lib.memopt_last_error()
+
+
+@pytest.mark.parametrize("fmt,H,D,q_len,tokens,splits", [
+    (1, 32, 128, 5, 131072, 16),   # the staged copy would pass 31 bits: room for the direct kernel's splits all the same
+    (0, 32, 128, 5, 131072, 16),
+    (1, 32, 128, 5, 130048, 0),    # one that fits: its size
+    (2, 8, 64, 100, 1024, 4),      # token-major codes are never staged
+])
+def test_multi_query_workspace_holds_the_splits(lib, fmt, H, D, q_len, tokens, splits):
+    """The workspace a multi-query call asks for holds the split partials the
+    direct kernel wants (splits * (D + 2) floats per query row and head)."""
+    import memopt_C
+    d = memopt_C.AttnDesc()
+    d.query = d.out = d.key_cache = d.value_cache = d.block_tables = d.context_lens = 256
+    d.key_scales = d.value_scales = 256
+    d.batch, d.q_len, d.num_heads, d.head_dim = 1, q_len, H, D
+    d.kv_format, d.block_size, d.num_kv_blocks = fmt, 16, tokens // 16
+    e = D if fmt == 0 else D // 2
+    d.kv_page_stride, d.kv_head_stride, d.kv_token_stride = 16 * H * e, e, H * e
+    d.max_blocks_per_seq, d.max_seq_len, d.window_size, d.causal = tokens // 16, tokens, tokens, 1
+    need = ctypes.c_int64()
+    ws = lib.memopt_attention_workspace_size
+    ws.argtypes = [ctypes.POINTER(memopt_C.AttnDesc), ctypes.POINTER(ctypes.c_int64)]
+    assert ws(ctypes.byref(d), ctypes.byref(need)) == OK
+    staged = (tokens // 16) * (H * 64 * D + 4) + H * 256
+    assert need.value == (q_len * H * splits * (D + 2) * 4 if splits else staged)

@@ -118,6 +118,18 @@ def test_noalloc_large_prefill_runs_unstaged(B, H, D, ctx, Lq, causal):
     assert_close(want, ref, what="regular (staged) prefill")
 
 
+@pytest.mark.parametrize("B,H,D,ctx,Lq", [(1, 2, 64, [512], 512), (1, 1, 128, [1100], 1100), (1, 4, 128, [3000], 20)])
+def test_noalloc_runs_the_regular_splits(B, H, D, ctx, Lq):
+    """Multi-query calls whose split partials fit the scratch run the regular
+    entry point's splits: equal bits."""
+    case = _pages_case(31 + Lq, B, H, D, ctx, Lq)
+    got, want, _ = _run_both(case, 1 << 20, 1 << 20, 4, True)
+    assert torch.equal(got, want)
+    q, pages, bt, cl = case
+    assert_close(got, O.paged_attention_int4(q, pages, bt, cl, 1 << 20, 1 << 20, num_sink_tokens=4, causal=True),
+                 what="noalloc")
+
+
 def test_noalloc_prepared_attention_and_limit():
     """PreparedAttention(no_alloc=True) holds no workspace and matches the
     regular call; partials past the scratch (forced splits) are refused."""
