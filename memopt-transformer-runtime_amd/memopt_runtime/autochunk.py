@@ -71,18 +71,19 @@ def autochunk_prefill(cache: PagedKVCache, seq_id: int, query: torch.Tensor, key
     # uploaded in one copy that nothing waits for; a chunk then costs its
     # launches. (Built chunk by chunk, the host took 177 us per 512-token
     # chunk, four times the kernels' time.) A pool without room for the whole
-    # prompt takes the chunks that fit, then raises.
-    n_fit = S
+    # prompt takes the chunks that fit, then raises. Fewer key rows than
+    # queries leave the later chunks' queries at the end of what is written.
+    rows = n_fit = min(S, keys.shape[0])
     try:
-        cache.reserve(seq_id, S)
+        cache.reserve(seq_id, rows)
     except RuntimeError:
-        n_fit = _whole_chunks(cache, seq_id, S, chunk_tokens)
+        n_fit = _whole_chunks(cache, seq_id, rows, chunk_tokens)
         cache.reserve(seq_id, n_fit)
-    index = cache.prompt_indices(seq_id, n_fit, [start + min(S, s0 + chunk_tokens) for s0 in
-                                                 range(0, n_fit, chunk_tokens)])
+    index = cache.prompt_indices(seq_id, n_fit, [start + min(rows, s0 + chunk_tokens) for s0 in
+                                                 range(0, S if n_fit == rows else n_fit, chunk_tokens)])
     for i, s0 in enumerate(range(0, S, chunk_tokens)):
         s1 = min(S, s0 + chunk_tokens)
-        cache.reserve(seq_id, s1 - s0)  # raises at the first chunk past n_fit
+        cache.reserve(seq_id, min(s1, rows) - min(s0, rows))  # raises at the first chunk past n_fit
         n = start + s1
         cache.write_rows([seq_id], keys[s0:s1], values[s0:s1], index.slots[s0:s1])
         memopt_C.PreparedAttention(query[s0:s1].unsqueeze(0), k_pool, v_pool,

@@ -156,7 +156,7 @@ class PagedKVCache:
         """Index tensors of the sequence's next ``tokens`` positions (reserved
         already) for calls that end at context lengths ``ends``: one upload,
         for use on the current stream."""
-        pages = self._pages[seq_id]
+        pages = self._pages[seq_id] or [-1]  # (a call's block table is never empty)
         slots = _slots_array(pages, self._len[seq_id], tokens, self.block_size)
         dev = upload_indices(np.concatenate([slots, pages, ends]), self.device)
         m = tokens + len(pages)

@@ -1,6 +1,6 @@
 """autochunk_prefill where the pool cannot hold the whole prompt: the chunks
 that fit are written and attended, then the call raises; and a shorter prompt
-appended after them."""
+appended after them. And where there are fewer key rows than queries."""
 import numpy as np
 import pytest
 import torch
@@ -30,3 +30,26 @@ def test_autochunk_out_of_pages():
     cache.free_sequence(0)
     assert memopt_C.free_blocks_count() == 14
     assert np.unique(memopt_C.allocate_blocks(14)).size == 14
+
+
+@pytest.mark.parametrize("held,rows", [(0, 25), (30, 25), (30, 0), (0, 0)])
+def test_autochunk_fewer_keys_than_queries(held, rows):
+    """Queries past the last key row: each chunk writes the rows it has, and its
+    queries end at the context written so far, as with append and an attention
+    call per chunk."""
+    import memopt_runtime as R
+    H, D, S, C = 2, 64, 40, 10
+    q, k, v = (torch.randn(S, H, D, device=dev(), dtype=torch.float16) for _ in range(3))
+    cache = R.PagedKVCache(14, H, D, kv_format="int4")
+    for s in (0, 1):
+        cache.add_sequence(s)
+        cache.append([s], k[None, :held], v[None, :held])
+    out = R.autochunk_prefill(cache, 0, q, k[:rows], v[:rows], window_size=64, num_sink_tokens=4, chunk_tokens=C)
+    assert cache.length(0) == held + rows
+    for s0 in range(0, S, C):
+        cache.append([1], k[None, s0:min(s0 + C, rows)], v[None, s0:min(s0 + C, rows)])
+        bt, ctx, _ = R.attention_inputs(cache, [1])
+        want = memopt_C.dynamic_sparse_attention(q[None, s0:s0 + C], *cache.key_value_pools(), bt, ctx,
+                                                 held + s0 + C, 64, num_sink_tokens=4, causal=True)
+        assert torch.equal(out[s0:s0 + C], want[0])
+    assert len(cache.pages(0)) == len(cache.pages(1))
