@@ -37,6 +37,14 @@ def _slots_array(pages: Sequence[int], start: int, count: int, block_size: int) 
     return page * block_size + pos % block_size
 
 
+def _int32(values: np.ndarray) -> np.ndarray:
+    """``values`` as int32; a slot past int32 (a pool of 2^31 tokens and more)
+    raises, where numpy's cast would wrap it to a slot that the kernels skip."""
+    if values.size and values.max() > np.iinfo(np.int32).max:
+        raise OverflowError(f"index {int(values.max())} out of bounds for int32")
+    return values.astype(np.int32)
+
+
 def upload_indices(values: np.ndarray, device: torch.device) -> torch.Tensor:
     """int32 copy of ``values`` on ``device``, ordered on the current stream
     and not waited for: from pinned memory, whose block torch's host allocator
@@ -44,7 +52,7 @@ def upload_indices(values: np.ndarray, device: torch.device) -> torch.Tensor:
     work queued before it, so the host could not run ahead of the GPU.) For
     tensors that the current stream alone uses."""
     host = torch.empty(values.shape, dtype=torch.int32, pin_memory=True)
-    host.numpy()[...] = values
+    host.numpy()[...] = _int32(values)
     return host.to(device, non_blocking=True)
 
 
@@ -150,7 +158,7 @@ class PagedKVCache:
     def slot_mapping(self, seq_ids: Sequence[int], new_tokens: int) -> torch.Tensor:
         """int32 slots of the next ``new_tokens`` positions of each sequence (sequence-major)."""
         slots = [_slots_array(self._pages[s], self._len[s], new_tokens, self.block_size) for s in seq_ids]
-        return torch.from_numpy(np.concatenate(slots or [np.empty(0)]).astype(np.int32)).to(self.device)
+        return torch.from_numpy(_int32(np.concatenate(slots or [np.empty(0)]))).to(self.device)
 
     def prompt_indices(self, seq_id: int, tokens: int, ends: Sequence[int]) -> "PromptIndices":
         """Index tensors of the sequence's next ``tokens`` positions (reserved

@@ -19,6 +19,18 @@ def test_slots_for(start, count):
         kv.slots_for([7, -1, 9], 3, 20, 16)
 
 
+def test_slots_past_int32_raise(monkeypatch):
+    """The last slot int32 holds, and the next one: an error, not a wrapped slot."""
+    import torch
+    _, kv = _modules()
+    monkeypatch.setattr(kv.PagedKVCache, "device", torch.device("cpu"))
+    cache = object.__new__(kv.PagedKVCache)
+    cache.block_size, cache._pages, cache._len = 16, {0: [2 ** 27 - 1, 2 ** 27]}, {0: 0}
+    assert cache.slot_mapping([0], 16)[-1] == 2 ** 31 - 1
+    with pytest.raises(OverflowError, match="2147483648"):
+        cache.slot_mapping([0], 17)
+
+
 def test_batch_allocation_keeps_fifo_order():
     M, _ = _modules()
     M.reset_pool()
