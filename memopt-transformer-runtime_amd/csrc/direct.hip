@@ -38,6 +38,7 @@
 // Waves merge through LDS; splits write fp32 partials that direct_merge_kernel
 // adds up (a launch of its own: the partials' workspace may hold anything).
 #include <algorithm>
+#include <cstdlib>
 
 #include "attention.hpp"
 #include "page_format.hpp"
@@ -671,6 +672,9 @@ static int direct_qb(const memopt_attn_desc &d) { return d.q_len <= 16 ? 1 : 2; 
 //    against 92; 8 of 64, 6000 queries, window 4096: 87 against 109 / 103
 //    against 110; 8 of 128, 8000 queries, window 2048: 123 against 86).
 static bool direct_faster(const memopt_attn_desc &d) {
+  // (MEMOPT_MULTI_QUERY_PATH=staged or =direct takes one path for every call,
+  // so that tests reach both at any size.)
+  if (const char *e = std::getenv("MEMOPT_MULTI_QUERY_PATH")) return *e == 'd';
   const int64_t q = d.q_len, tiles = (q + 127) / 128 * d.num_heads * d.batch;
   if (q <= 192 || tiles <= 128) return true;
   // Pairs of one sequence at the longest context the block table holds.
@@ -700,7 +704,7 @@ bool direct_supported(const memopt_attn_desc &d) {
   auto al = [](const void *x, int64_t a) { return ((uintptr_t)x & (uintptr_t)(a - 1)) == 0; };
   if (d.q_len < 2 || (d.head_dim != 64 && d.head_dim != 128) || d.num_kv_blocks <= 0) return false;
   if (!al(d.query, 16) || !al(d.out, 16)) return false;
-  if (d.kv_format != MEMOPT_KV_INT4_ROWS) return direct_faster(d) && prefill_supported(d);
+  if (d.kv_format != MEMOPT_KV_INT4_ROWS) return prefill_supported(d) && direct_faster(d);
   if (d.block_size % 16 != 0) return false;
   // 16-byte (D = 128) or 8-byte loads of a token's codes
   const int64_t a = d.head_dim / 8;

@@ -283,8 +283,9 @@ def test_config4_full_rows_int4_pages():
 
 
 def _prefill_with_env(env, *args, **kw):
-    """One attention call with the given environment overrides in place."""
+    """One attention call on the staged path with the given environment overrides in place."""
     import os
+    env = dict(env, MEMOPT_MULTI_QUERY_PATH="staged")
     old = {k: os.environ.get(k) for k in env}
     os.environ.update(env)
     try:

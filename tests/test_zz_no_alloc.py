@@ -19,6 +19,12 @@ pytestmark = pytest.mark.gpu
 SCRATCH_BYTES = 4 << 20
 
 
+@pytest.fixture
+def staged(monkeypatch):
+    """Multi-query calls of these sizes take the direct kernel by themselves."""
+    monkeypatch.setenv("MEMOPT_MULTI_QUERY_PATH", "staged")
+
+
 def _entry_points():
     import memopt_C as M
     f = M._lib.memopt_paged_attention_noalloc
@@ -73,7 +79,7 @@ def test_noalloc_split_k_decode_two_calls():
                      what="noalloc decode")
 
 
-def test_noalloc_staged_prefill_two_calls():
+def test_noalloc_staged_prefill_two_calls(staged):
     first = _pages_case(3, 1, 2, 128, [512], 128)
     second = _pages_case(4, 1, 2, 128, [256], 64)
     for case, W in ((first, 256), (second, 100)):
@@ -85,7 +91,7 @@ def test_noalloc_staged_prefill_two_calls():
                      what="noalloc prefill")
 
 
-def test_noalloc_decode_after_staged_prefill():
+def test_noalloc_decode_after_staged_prefill(staged):
     """A staged multi-query call writes its K/V over the scratch the split-K
     partials use; the decode after it must still merge its splits (its
     arrival counters live in the scratch's last 64 KiB, which nothing else
@@ -104,7 +110,7 @@ def test_noalloc_decode_after_staged_prefill():
 
 @pytest.mark.parametrize("B,H,D,ctx,Lq,causal", [(2, 4, 128, [3835, 696], 2, False),
                                                  (3, 2, 64, [5243, 266, 2961], 120, True)])
-def test_noalloc_large_prefill_runs_unstaged(B, H, D, ctx, Lq, causal):
+def test_noalloc_large_prefill_runs_unstaged(B, H, D, ctx, Lq, causal, staged):
     """A multi-query call whose staged K/V would not fit the static scratch
     runs the kernel that dequantizes into LDS itself (no scratch): its output
     and the regular entry point's (staged) are both within the tests'
