@@ -355,7 +355,8 @@ static int paged_attention(const memopt_attn_desc &d, bool unsplit_ok, void *str
                : cnt       ? cnt
                            : (unsigned long long *)(p.ws_ml + (int64_t)d.batch * d.num_heads * splits * 2);
     p.tag = next_decode_tag();
-    return launch_decode_int4(p, d.batch, d.head_dim, d.kv_format == MEMOPT_KV_INT4 ? MEMOPT_SCALE_F16 : d.scale_dtype, s);
+    return launch_decode_int4(p, d.batch, d.head_dim, d.kv_format == MEMOPT_KV_INT4 ? MEMOPT_SCALE_F16 : d.scale_dtype,
+                              max_pages_visited(d), s);
   }
 
   if (use_decode_fp16(d)) {

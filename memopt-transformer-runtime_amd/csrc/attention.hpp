@@ -60,7 +60,7 @@ struct DecodeParams {
   int32_t pages;                // 1: this build's INT4 page format (page_format.hpp)
   int32_t M, H, W, sinks, splits;
   int32_t bs;           // tokens per page (fp16 pools; a multiple of 16)
-  int32_t hc;           // heads per cluster (token-major codes; 1: grid order)
+  int32_t B, hc, groups;  // token-major codes: sequences, heads per cluster (1: grid order), clusters per sequence
   float qk_scale_log2;  // (1/sqrt(D)) * log2(e)
   float *ws_o;          // [B, H, splits, D] (splits > 1)
   float *ws_ml;         // [B, H, splits, 2]
@@ -188,8 +188,9 @@ __device__ __forceinline__ void decode_epilogue(const DecodeParams &p, int64_t b
 
 // Split count used by the decode kernels for this launch shape.
 int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool int4);
-// Launches the split-K INT4 decode kernel (splits merged in-kernel).
-int launch_decode_int4(const DecodeParams &p, int32_t batch, int32_t D, int32_t scale_dtype,
+// Launches the split-K INT4 decode kernel (splits merged in-kernel); `pages`:
+// the pages a sequence may visit.
+int launch_decode_int4(const DecodeParams &p, int32_t batch, int32_t D, int32_t scale_dtype, int32_t pages,
                        hipStream_t stream);
 
 // Launches the split-K fp16-pool decode kernel (splits merged in-kernel).

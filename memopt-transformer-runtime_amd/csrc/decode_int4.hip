@@ -136,15 +136,26 @@ __global__ __launch_bounds__(NW * 64) void decode_int4_kernel(const DecodeParams
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Head clusters (head_cluster): with hc > 1, workgroup i takes head i / 8 %
-  // hc of the cluster of its XCD (i % 8).
+  // Head clusters (cluster_heads): grid (8 hc, groups, ceil(units / 8)) over
+  // the units u = (b, split), or (8 hc, 1, units * groups / 8) for fewer than
+  // 8 units. blockIdx.x is 8 * head of the cluster + XCD in both.
   int32_t b = blockIdx.z, h = blockIdx.y, split = blockIdx.x;
   if (p.hc > 1) {
-    const int32_t id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), slot = id >> 3;
-    const int32_t cl = slot / p.hc * 8 + (id & 7), per = p.H / p.hc, u = cl / per;  // u = (b, split)
-    h = (cl - u * per) * p.hc + slot % p.hc;
-    b = u / p.splits;
-    split = u - b * p.splits;
+    const int32_t xcd = blockIdx.x & 7;
+    int32_t grp = blockIdx.y, u = blockIdx.z * 8 + ((xcd - grp) & 7);
+    if ((int32_t)gridDim.y != p.groups) {
+      const int32_t cl = blockIdx.z * 8 + xcd;
+      u = cl / p.groups;
+      grp = cl - u * p.groups;
+    }
+    h = grp * p.hc + (blockIdx.x >> 3);
+    b = u;
+    split = 0;
+    if (p.splits > 1) {
+      b = u / p.splits;
+      split = u - b * p.splits;
+    }
+    if (b >= p.B) return;  // the last eight units are not all there
   }
   const int t = lane >> 2, c = lane & 3;
   const int g = (c * DPL) / 64;  // scale group of this lane's dims
@@ -593,19 +604,35 @@ int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool 
 // Heads of a cluster of the token-major kernel. A token's codes are D / 2
 // bytes per head and its scales D / 64 floats, so neighbouring heads share
 // 128-byte lines; workgroups are dealt to the 8 XCDs round-robin, and heads
-// on different XCDs fetch such a line once per L2. The largest power-of-two
-// fraction of H whose clusters deal out evenly over the XCDs (1: none). With
-// the double buffering, 16 sequences of 4096 tokens x 32 heads of 128 (302 MB)
-// went from 139 to 96 us (fetching 321 MB), 8 heads of 64 from 27 to 15. What
-// is left is throughput below the L1s: per page and head the loads touch 64
-// pieces of lines (the page layout: 18), and neither more pages in flight
-// nor more waves changed it.
-static int32_t head_cluster(int32_t batch, int32_t splits, int32_t H) {
-  for (int32_t hc = H; hc > 1; hc /= 2) {
-    if ((int64_t)batch * splits * (H / hc) % 8 == 0) return hc;
-    if (hc % 2) break;
+// on different XCDs fetch such a line once per L2. At most 8 heads, a
+// multiple of those that share a line of codes where H has such a divisor,
+// and a unit's clusters on different XCDs: with all heads of a unit on one
+// (a few per cent faster on equal lengths: 8 sequences of 4096 tokens x 32
+// heads of 128 37.7 us, in eights 39.2, unclustered 62) a long sequence in a
+// batch of short ones is drawn through one XCD (8 sequences x 40 heads, one
+// of 16384 tokens, the rest 500: unclustered 82 us, all heads 100, eights 57;
+// the mean of four random placements of three long ones among 32: 228, 190,
+// 168). A cluster's heads follow each other on their XCD: a stride between
+// them puts them on the same shader engine (62 us instead of 37 for the two
+// long ones of 16 x 12 heads of 64). Fewer than 8 units are clustered where
+// the clusters deal out evenly, and calls of fewer than 6000 blocks (16 tokens
+// of one head) not at all: the caches hold their lines, and finding its unit
+// costs a workgroup 0.1 to 0.5 us (16 sequences of 120 tokens x 40 heads of 128,
+// 5120 blocks: 11.4 us, clustered 11.6; 200 tokens x 32 heads, 6656 blocks:
+// 11.9 and 10.1; of 64, 16 x 20 heads, 5440 blocks 7.5 and 7.5, 8000 10.8 and
+// 8.5). With the double buffering, 16 sequences of 4096 tokens x 32 heads of
+// 128 (302 MB) went from 139 to 89 us, 8 heads of 64 from 20 to 13.5. What is left is throughput below the L1s: per page and
+// head the loads touch 64 pieces of lines (the page layout: 18), and neither
+// more pages in flight nor more waves changed it.
+static int32_t cluster_heads(int64_t units, int32_t H, int32_t D, int64_t blocks) {
+  if (blocks < 6000) return 1;
+  const int32_t line = 256 / D;
+  int32_t best = 1;
+  for (int32_t hc = 2; hc <= 8 && hc <= H; ++hc) {
+    if (H % hc != 0 || (units < 8 && units * (H / hc) % 8 != 0)) continue;
+    if (hc % line == 0 || best % line != 0) best = hc;
   }
-  return 1;
+  return (units + 7) / 8 * (H / best) <= 65535 ? best : 1;  // (grid dimensions)
 }
 
 template <int D, typename ST>
@@ -627,12 +654,17 @@ static void launch_shape(const DecodeParams &p, dim3 grid, DecodeShape sh, hipSt
 #undef MEMOPT_DECODE_CASE
 }
 
-int launch_decode_int4(const DecodeParams &params, int32_t batch, int32_t D, int32_t scale_dtype,
+int launch_decode_int4(const DecodeParams &params, int32_t batch, int32_t D, int32_t scale_dtype, int32_t pages,
                        hipStream_t stream) {
   DecodeParams p = params;
-  p.hc = p.pages ? 1 : head_cluster(batch, p.splits, p.H);
   const DecodeShape sh = decode_shape();
-  const dim3 grid(p.splits, p.H, batch);
+  const int64_t units = (int64_t)batch * p.splits;
+  p.B = batch;
+  p.hc = p.pages ? 1 : cluster_heads(units, p.H, D, (int64_t)batch * p.H * pages);
+  p.groups = p.H / p.hc;
+  dim3 grid(p.splits, p.H, batch);
+  if (p.hc > 1 && units >= 8) grid = dim3(8 * p.hc, p.groups, (unsigned)((units + 7) / 8));
+  else if (p.hc > 1) grid = dim3(8 * p.hc, 1, (unsigned)(units * p.groups / 8));
   if (D == 128 && scale_dtype == MEMOPT_SCALE_F16)
     launch_shape<128, half_t>(p, grid, sh, stream);
   else if (D == 128)

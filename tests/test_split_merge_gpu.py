@@ -78,8 +78,8 @@ def test_captured_split_decode_replays():
 
 @pytest.mark.parametrize("B,H", [(1, 1), (1, 8), (2, 12), (3, 5), (8, 3), (16, 6), (1, 40)])
 def test_token_major_head_clusters(B, H):
-    """Head counts and batches whose clusters cover all heads, a fraction, or
-    none: every (sequence, head) is computed once, in its place."""
+    """Short calls (unclustered) over head counts and batches: every (sequence,
+    head) is computed once, in its place."""
     rng = np.random.default_rng(B * 100 + H)
     ctx = [int(x) for x in rng.integers(1, 90, B)]
     q, k, v, bt, cl = _case(B + H, B, H, 64, ctx)
@@ -88,3 +88,29 @@ def test_token_major_head_clusters(B, H):
     got = memopt_C.dynamic_sparse_attention(to_dev(q), to_dev(kq), to_dev(vq), to_dev(bt), to_dev(cl), 128, 128,
                                             key_scales=to_dev(ks), value_scales=to_dev(vs), kv_layout="token_major")
     assert_close(got, want, what=f"{B} x {H} token-major heads")
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,splits", [(1, 16, 1), (3, 32, 1), (2, 20, 2), (7, 8, 1), (8, 3, 1), (9, 12, 1),
+                                        (5, 7, 3), (16, 40, 1), (1, 64, 8), (2, 1, 5)])
+def test_token_major_head_clusters_of_long_calls(B, H, splits, D, monkeypatch):
+    """Calls whose block tables hold enough pages for head clusters (most of
+    them unlinked here): fewer than 8 (sequence, split) units, 8, numbers
+    between multiples of 8; cluster sizes 1 to 8, one to eight per unit."""
+    monkeypatch.setenv("MEMOPT_DECODE_SPLITS", str(splits))
+    rng = np.random.default_rng(B * 100 + H)
+    ctx = [int(x) for x in rng.integers(1, 90, B)]
+    q, k, v, bt, cl = _case(B + H, B, H, D, ctx)
+    M = 6000 // (B * H) + 2
+    wide = np.full((B, M), -1, np.int32)
+    at = 7 * np.arange(bt.shape[1]) % M                # pages spread over the table, so over the splits
+    assert len(set(at)) == bt.shape[1]
+    at.sort()
+    wide[:, at] = bt
+    cl = np.array([16 * int(at[(c - 1) // 16]) + (c - 1) % 16 + 1 for c in ctx], np.int32)
+    (kq, ks), (vq, vs) = O.quantize_int4(k), O.quantize_int4(v)
+    n = 16 * M
+    want = O.paged_attention(q, O.dequantize_int4(kq, ks), O.dequantize_int4(vq, vs), wide, cl, n, n)
+    got = memopt_C.dynamic_sparse_attention(to_dev(q), to_dev(kq), to_dev(vq), to_dev(wide), to_dev(cl), n, n,
+                                            key_scales=to_dev(ks), value_scales=to_dev(vs), kv_layout="token_major")
+    assert_close(got, want, what=f"{B} x {H} token-major heads of {D} in {splits} splits")
