@@ -37,6 +37,7 @@
 //    block-table entries < 0 or >= num_kv_blocks are skipped, and split-K
 //    partials (m, l, o) are merged by the last split of each (b, h) to
 //    finish (decode_epilogue).
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 
@@ -567,28 +568,37 @@ static DecodeShape decode_shape() {
 }
 
 // Splits of a decode over `units` (b, h) pairs, measured for both formats
-// over 32 to 384 units and 1500 to 16000 tokens (MI355X, 256 CUs):
-//  * fewer units than CUs: as many splits as keep the grid within two
-//    workgroups per CU; fp16, whose loads fill a CU's share alone, within one
-//    up to a quarter of the CUs, and 3 splits above half of them. A grid past
-//    that runs in uneven rounds: 120 units of 6000 tokens, INT4 in 7, 4
-//    splits 24.9, 20.8 us, fp16 70.9, 65.0; 64 units fp16 in 12, 4 40.8, 34.7;
-//    200 units INT4 in 4, 2 37.0, 31.5, fp16 in 4, 3 118.6, 107.9. Fewer lose
-//    on unequal lengths (160 units of 2000 to 5000 tokens, fp16 in 5, 3, 1
-//    splits 54.6, 53.9, 75.8);
+// over 32 to 384 units and 1500 to 16000 tokens, equal lengths and lengths of
+// which one, some or none reach the longest (MI355X, 256 CUs):
+//  * INT4 up to half the CUs: as many as keep the grid within two workgroups
+//    per CU; a grid past that runs in uneven rounds (120 units of 6000 tokens
+//    24.9 us in 7, 20.8 in 4);
+//  * INT4 above that: three workgroups per CU. Fewer win on equal lengths (200
+//    units of 6000 tokens 37.0 us in 4, 31.5 in 2) and lose more on unequal
+//    ones, where the longest sequence's workgroups go on alone (192 units, the
+//    longest of 12000 tokens: up to 1.35 times as long in 2 as in 4);
+//  * fp16, whose loads fill a CU's share alone, up to a fifth of the CUs: one
+//    workgroup per CU (40 units of 6000 tokens 45 us in 20, 26 in 6);
+//  * fp16 above that: two, and at least 6 splits (64 units 0.78 of the time
+//    of 12 splits in 8, and at most 0.88 on unequal lengths, in 4 0.80 and
+//    1.07; 66 units of 6000 tokens 39 us in 7, 51 in 4; 120 67 in 6, 68 in 4;
+//    160 units 0.90 and 1.02 of the time of 5 splits in 6, 0.96 and 1.20 in 3);
 //  * 256 to 511 units: 2 (unsplit is up to 8 % faster on equal lengths, but
 //    10 % slower on lengths from a third to the whole of 4000 tokens);
 //  * at least 4 page batches per wave, and INT4 contexts of up to 64 pages are
 //    not split: the merge and the cleared workspace cost more than the pages
-//    they save (64 pages, 8 heads of 64: 6.5 us unsplit, 8.3 in 2; 94 pages,
-//    32 heads of 128: 10.7 against 9.2 and 2 for the clearing).
+//    they save (8 heads of 64: 48 pages 6.0 us unsplit, 6.9 in 2; 64 pages 6.8
+//    and 7.3; 80 pages 7.7 and 7.8; 32 heads of 128: 7.4 and 8.3, 8.7 and 8.7,
+//    9.9 and 9.4, and 2 for the clearing).
 int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool int4) {
   const int64_t units = (int64_t)batch * heads;
   if (units <= 0) return 1;
   const DecodeShape sh = decode_shape();
   const int64_t cus = compute_units();
-  int64_t s = units < cus ? 2 * cus / units : (2 * cus + units - 1) / units;
-  if (!int4 && units < cus) s = 4 * units <= cus ? cus / units : 2 * units <= cus ? s : 3;
+  int64_t s;
+  if (units >= cus) s = (2 * cus + units - 1) / units;
+  else if (int4) s = 2 * units <= cus ? 2 * cus / units : (3 * cus + units - 1) / units;
+  else s = 5 * units <= cus ? cus / units : std::max<int64_t>(6, 2 * cus / units);
   const int64_t cap = max_pages_visited / (4LL * sh.nw * sh.u);
   if (s > cap) s = cap;
   if (int4 && max_pages_visited <= 64) s = 1;

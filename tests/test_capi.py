@@ -187,3 +187,25 @@ def test_multi_query_workspace_holds_the_splits(lib, fmt, H, D, q_len, tokens, s
     assert ws(ctypes.byref(d), ctypes.byref(need)) == OK
     staged = (tokens // 16) * (H * 64 * D + 4) + H * 256
     assert need.value == (q_len * H * splits * (D + 2) * 4 if splits else staged)
+
+
+@pytest.mark.parametrize("fmt,units,tokens,splits", [
+    (1, 8, 1024, 1), (1, 8, 6000, 11), (1, 120, 6000, 4), (1, 128, 6000, 4), (1, 129, 6000, 6), (1, 160, 6000, 5),
+    (1, 192, 6000, 4), (1, 255, 6000, 4), (1, 256, 6000, 2), (1, 511, 6000, 2), (1, 512, 6000, 1),
+    (0, 40, 6000, 6), (0, 51, 6000, 5), (0, 52, 6000, 9), (0, 64, 6000, 8), (0, 96, 6000, 6), (0, 200, 6000, 6),
+    (0, 255, 6000, 6), (0, 256, 6000, 2), (0, 200, 1500, 2), (0, 200, 900, 1),
+])
+def test_decode_split_counts(lib, fmt, units, tokens, splits):
+    """Split counts of a decode on 256 CUs, from the workspace they need."""
+    import memopt_C
+    d = memopt_C.AttnDesc()
+    d.query = d.out = d.key_cache = d.value_cache = d.block_tables = d.context_lens = 256
+    d.batch, d.q_len, d.num_heads, d.head_dim = 1, 1, units, 128
+    d.kv_format, d.block_size, d.num_kv_blocks = fmt, 16, 4096
+    d.kv_page_stride, d.kv_head_stride, d.kv_token_stride = 16 * units * 128, 128, units * 128
+    d.max_blocks_per_seq, d.max_seq_len, d.window_size = -(-tokens // 16), tokens, tokens
+    need = ctypes.c_int64()
+    ws = lib.memopt_attention_workspace_size
+    ws.argtypes = [ctypes.POINTER(memopt_C.AttnDesc), ctypes.POINTER(ctypes.c_int64)]
+    assert ws(ctypes.byref(d), ctypes.byref(need)) == OK
+    assert need.value == (units * splits * (128 + 2) * 4 + 8 * units if splits > 1 else 0)
