@@ -38,6 +38,7 @@
 // Waves merge through LDS; splits write fp32 partials that direct_merge_kernel
 // adds up (a launch of its own: the partials' workspace may hold anything).
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "attention.hpp"
@@ -646,37 +647,48 @@ __global__ __launch_bounds__(256) void direct_merge_kernel(const DirectParams p,
 static int direct_qb(const memopt_attn_desc &d) { return d.q_len <= 16 ? 1 : 2; }
 
 // Where the direct kernel beats the staged path (staging and attention
-// launches together, both sides measured with 8 to 40 heads, batches of 1 to
-// 16, contexts of 300 to 16384 tokens, over pages / fp16 pools):
-//  * up to 192 queries, whatever the batch: staging costs about what 128
-//    queries compute (8 sequences of 2000 tokens x 32 heads, 128 queries: 67
-//    against 142 us / 146 against 177; 4 of 8192, 192 queries: 186 against
-//    302 / 335 against 374; 4 of 2048, 256 queries: 65 against 76 / 99
-//    against 94);
-//  * up to 128 tiles of 128 queries, which leave half of the CUs idle on the
-//    staged path (32 heads, 512 queries over 2048 tokens: 51 against 54 us
-//    over pages, over 16384: 244 against 372);
-//  * little work per call, where the staging launch and the ramp of the long
-//    tiles weigh more than the staged path's faster inner loop: by (query,
-//    key) pairs over all heads, up to 32 / 24 million at D = 128 (25 M, 8
-//    heads x 2500 queries: 44 against 74 us / 47 against 74; 34 M, 32 heads x
-//    1024 queries, window 1024: 44 against 46 / 51 against 47; 50 M: 64
-//    against 55 / 74 against 56) and 110 / 70 million at D = 64 (83 M, 12
-//    heads x 4413 queries, window 2048: 59 against 68 / 70 against 68; 154 M:
-//    101 against 88 / 121 against 94);
-//  * few heads over long contexts: with at most two of its workgroups per CU
-//    the staged path takes as long as its longest tile, about 1.4 us per 64
-//    keys and 10 us, whatever the rest of the grid does, and the direct
-//    kernel 8 us and the pairs at its rate (8 heads of 128, 4000 causal
-//    queries: 83 against 106 us / 96 against 105, of 64: 55 against 91 / 62
-//    against 92; 8 of 64, 6000 queries, window 4096: 87 against 109 / 103
-//    against 110; 8 of 128, 8000 queries, window 2048: 123 against 86).
+// launches together). Both times are estimated, in us, from sums fitted to
+// both paths timed on 61000 random calls over pages and fp16 pools (1 to 40
+// heads, 1 to 16 sequences, 2 to 8192 queries, 20 to 32768 tokens, windows,
+// causal or not, equal and unequal lengths; median error 4 to 6 %):
+//  * a workgroup takes a fixed time and one per key it visits, and `both`
+//    more of that when a second one shares its CU; past two per CU the grid
+//    runs in rounds, whose last one counts `ramp` in full. A causal staged
+//    grid ends with its longest tile;
+//  * staging a (token, head, dim) of K and V costs `stage` per million;
+//  * each block of 32 queries reads its keys again: with many heads at once
+//    these reads pass the caches, at 150 / sqrt(MB of K and V) MB per us
+//    (16 sequences of 2277 fp16 tokens x 32 heads of 128, 486 queries: 1571
+//    us, staged 576; 178 queries on 3568 tokens x 32 heads of 64 525 and 371).
+// The estimates decide above 128 queries and 128 tiles (fewer tiles leave half
+// of the CUs idle on the staged path). Fixed numbers of queries, tiles and
+// (query, key) pairs, which drew the line before, lost 8 to 45 % on 266 of
+// those calls (4 x 4 heads of 128, 3540 queries in a 512-token window, not
+// causal: 50 us, staged 40; 1 x 32 heads, fp16, 1687 causal queries: 51 and
+// 44; 2 x 40 heads, 530 queries: 49 and 43); on 34900 further random calls
+// this rule loses more than 8 % on 31.
+struct PathCost {
+  double block, key, both;       // direct: per block, per thousand keys
+  double tile, tile_key, tile_both, stage;
+};
+static const PathCost kPathCost[2][2] = {
+    // D = 64, 128
+    {{1.4, 6.2, 0.39, 2.4, 21.5, 0.30, 0.84}, {2.7, 7.2, 0.87, 6.6, 25.3, 0.42, 0.70}},  // pages
+    {{1.3, 7.5, 0.41, 2.4, 21.5, 0.30, 1.16}, {1.9, 8.1, 1.18, 6.6, 25.3, 0.42, 0.92}},  // fp16 pools
+};
+
+// Time of n equal workgroups in units of one alone on its CU.
+static double grid_time(double n, double both, double ramp) {
+  const double x = n / compute_units(), fill = 1.0 + both * std::min(1.0, std::max(0.0, x - 1.0));
+  return fill * (x <= 2.0 ? 1.0 : (1.0 - ramp) * x / 2 + ramp * std::ceil(x / 2));
+}
+
 static bool direct_faster(const memopt_attn_desc &d) {
   // (MEMOPT_MULTI_QUERY_PATH=staged or =direct takes one path for every call,
   // so that tests reach both at any size.)
   if (const char *e = std::getenv("MEMOPT_MULTI_QUERY_PATH")) return *e == 'd';
-  const int64_t q = d.q_len, tiles = (q + 127) / 128 * d.num_heads * d.batch;
-  if (q <= 192 || tiles <= 128) return true;
+  const int64_t q = d.q_len, heads = (int64_t)d.num_heads * d.batch, tiles = (q + 127) / 128 * heads;
+  if (q <= 128 || tiles <= 128) return true;
   // Pairs of one sequence at the longest context the block table holds.
   const int64_t T = (int64_t)d.max_blocks_per_seq * d.block_size;
   const int64_t W = std::min<int64_t>(effective_window(d.window_size, d.max_seq_len), T);
@@ -685,13 +697,21 @@ static bool direct_faster(const memopt_attn_desc &d) {
     const int64_t lo = std::max<int64_t>(0, T - q), full = std::max(lo, std::min(W, T));
     pairs = (full - lo) * (full + lo + 1) / 2 + (T - full) * W;
   }
-  const bool pages = d.kv_format == MEMOPT_KV_INT4;
-  const bool d128 = d.head_dim == 128;
-  const double mpairs = 1e-6 * (double)pairs * d.num_heads * d.batch;
-  if (mpairs <= (d128 ? (pages ? 32.0 : 24.0) : (pages ? 110.0 : 70.0))) return true;
-  const double rate = d128 ? (pages ? 0.85 : 0.68) : (pages ? 1.65 : 1.38);  // million pairs per us
-  const double keys = (double)std::min(T, d.causal ? W + 127 : W);           // of the longest tile
-  return tiles <= 2 * compute_units() && 8.0 + mpairs / rate < 0.9 * (10.0 + 1.4 * keys / 64);
+  const bool pages = d.kv_format == MEMOPT_KV_INT4, clip = W < T, sinks = clip && d.num_sink_tokens > 0;
+  const PathCost &c = kPathCost[pages ? 0 : 1][d.head_dim == 128];
+  // Thousands of keys a block or tile visits, ragged edges included.
+  const double mean = (double)pairs / (double)q;
+  const double keys = 1e-3 * (mean + (!d.causal ? 0 : clip ? 24 : 8) + (sinks ? 16 : 0));
+  const double tile_keys = 1e-3 * (mean + (!d.causal ? 0 : clip ? 96 : 32) + (sinks ? 64 : 0));
+  const double longest = 1e-3 * (double)(d.causal ? std::min(T, W + 127) : W);
+  const double blocks = (double)((q + 31) / 32);
+  const double melems = 1e-6 * (double)(std::min(T, d.causal ? q + W : W) * heads * d.head_dim);  // K and V staged
+  double direct = 4.5 + (c.block + c.key * keys) * grid_time(blocks * heads, c.both, 0.42);
+  const double staged = 10.0 + (c.tile + c.tile_key * tile_keys) * grid_time((double)tiles, c.tile_both, 0.22) +
+                        16.5 * (longest - tile_keys) + c.stage * melems;
+  const double passes = blocks * std::min(1.0, heads / 128.0), mb = melems * (pages ? 1.125 : 4.0);
+  if (passes > 1.0) direct = std::max(direct, passes * mb * std::sqrt(mb) / 150.0);
+  return direct < 0.94 * staged;
 }
 
 static int64_t direct_query_blocks(const memopt_attn_desc &d) {

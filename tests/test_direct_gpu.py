@@ -143,6 +143,37 @@ def test_direct_rows_non_finite_scores(D, scale, n):
     assert_close(memopt_C.PreparedAttention(*args, no_alloc=True, **kw)(), got, what="no_alloc")
 
 
+@pytest.mark.parametrize("layout,B,H,D,n,Lq,W,causal,path", [
+    ("pages", 4, 4, 128, 3540, 3540, 512, False, "staged"),
+    ("fp16", 1, 32, 128, 1687, 1687, 512, True, "staged"),
+    ("fp16", 16, 32, 64, 3568, 178, 1 << 20, True, "staged"),      # the blocks' repeated reads pass the caches
+    ("pages", 1, 32, 128, 700, 700, 1 << 20, True, "direct"),
+    ("pages", 4, 12, 64, 1000, 500, 1 << 20, True, "direct"),
+    ("fp16", 2, 8, 128, 1024, 128, 1 << 20, False, "direct"),
+])
+def test_multi_query_path_by_estimate(layout, B, H, D, n, Lq, W, causal, path, monkeypatch):
+    """Calls far to either side of the line between the direct kernel and the
+    staged path run the faster one (equal bits), and both agree."""
+    g = torch.Generator(device=dev()).manual_seed(Lq)
+    nb = B * -(-n // 16)
+    k, v = (torch.randn((nb, 16, H, D), generator=g, device=dev(), dtype=torch.float16) for _ in range(2))
+    if layout == "pages":
+        memopt_C.init_pool(nb, 16, H, D, kv_format="int4")
+        memopt_C.write_cache(k.view(-1, H, D), v.view(-1, H, D), None,
+                             torch.arange(nb * 16, dtype=torch.int32, device=dev()))
+        k = v = memopt_C.get_int4_pages()
+    q = torch.randn((B, Lq, H, D), generator=g, device=dev(), dtype=torch.float16)
+    bt = torch.randperm(nb, generator=g, device=dev()).to(torch.int32).view(B, -1).contiguous()
+    cl = torch.full((B,), n, dtype=torch.int32, device=dev())
+    out = {}
+    for name in ("", "staged", "direct"):
+        if name:
+            monkeypatch.setenv("MEMOPT_MULTI_QUERY_PATH", name)
+        out[name] = memopt_C.dynamic_sparse_attention(q, k, v, bt, cl, n, W, causal=causal)
+    assert torch.equal(out[""], out[path]) and not torch.equal(out["staged"], out["direct"])
+    assert_close(out["direct"], out["staged"].cpu(), what="direct vs staged")
+
+
 def test_more_query_blocks_than_a_grid_dimension():
     """2097152 queries (65536 blocks of 32, one more than the direct kernel's
     grid takes) with little work per query: served, as any other length."""
