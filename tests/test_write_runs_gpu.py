@@ -17,6 +17,8 @@ pytestmark = pytest.mark.gpu
     [1] * 15 + [64],        # scattered tokens, then pages from token 15 on
     [16, 15, 16, 17, 100],
     [200],
+    [5, 16, 40, 31, 1] + [997] * 8,  # enough elements for pages from any token (1.5 M at D = 64)
+    [997] * 7 + [833],               # just too few
 ])
 def test_write_page_runs(D, lens):
     """Sequences back to back, each at the start of its own pages (permuted);
