@@ -37,14 +37,6 @@ def _slots_array(pages: Sequence[int], start: int, count: int, block_size: int) 
     return page * block_size + pos % block_size
 
 
-def _int32(values: np.ndarray) -> np.ndarray:
-    """``values`` as int32; a slot past int32 (a pool of 2^31 tokens and more)
-    raises, where numpy's cast would wrap it to a slot that the kernels skip."""
-    if values.size and values.max() > np.iinfo(np.int32).max:
-        raise OverflowError(f"index {int(values.max())} out of bounds for int32")
-    return values.astype(np.int32)
-
-
 def upload_indices(values: np.ndarray, device: torch.device) -> torch.Tensor:
     """int32 copy of ``values`` on ``device``, ordered on the current stream
     and not waited for: from pinned memory, whose block torch's host allocator
@@ -52,7 +44,7 @@ def upload_indices(values: np.ndarray, device: torch.device) -> torch.Tensor:
     work queued before it, so the host could not run ahead of the GPU.) For
     tensors that the current stream alone uses."""
     host = torch.empty(values.shape, dtype=torch.int32, pin_memory=True)
-    host.numpy()[...] = _int32(values)
+    host.numpy()[...] = values
     return host.to(device, non_blocking=True)
 
 
@@ -157,15 +149,24 @@ class PagedKVCache:
 
     def slot_mapping(self, seq_ids: Sequence[int], new_tokens: int) -> torch.Tensor:
         """int32 slots of the next ``new_tokens`` positions of each sequence (sequence-major)."""
-        slots = [_slots_array(self._pages[s], self._len[s], new_tokens, self.block_size) for s in seq_ids]
-        return torch.from_numpy(_int32(np.concatenate(slots or [np.empty(0)]))).to(self.device)
+        slots = [self._next_slots(s, new_tokens) for s in seq_ids]
+        return torch.from_numpy(np.concatenate(slots or [np.empty(0)]).astype(np.int32)).to(self.device)
+
+    def _next_slots(self, seq_id: int, count: int) -> np.ndarray:
+        """int64 slots of the sequence's next ``count`` positions; one past int32
+        (a pool of 2^31 tokens and more) raises, where the cast to int32 would
+        wrap it to a slot that the kernels skip."""
+        slots = _slots_array(self._pages[seq_id], self._len[seq_id], count, self.block_size)
+        if self.num_blocks * self.block_size > 2 ** 31 and count and slots.max() >= 2 ** 31:
+            raise OverflowError(f"slot {int(slots.max())} out of bounds for int32")
+        return slots
 
     def prompt_indices(self, seq_id: int, tokens: int, ends: Sequence[int]) -> "PromptIndices":
         """Index tensors of the sequence's next ``tokens`` positions (reserved
         already) for calls that end at context lengths ``ends``: one upload,
         for use on the current stream."""
         pages = self._pages[seq_id] or [-1]  # (a call's block table is never empty)
-        slots = _slots_array(pages, self._len[seq_id], tokens, self.block_size)
+        slots = self._next_slots(seq_id, tokens)
         dev = upload_indices(np.concatenate([slots, pages, ends]), self.device)
         m = tokens + len(pages)
         return PromptIndices(dev[:tokens], dev[tokens:m].unsqueeze(0), dev[m:])
@@ -186,8 +187,8 @@ class PagedKVCache:
             raise RuntimeError("append: keys batch != number of sequences")
         for s in seq_ids:
             self.reserve(s, T)
-        slots = upload_indices(np.concatenate([_slots_array(self._pages[s], self._len[s], T, self.block_size)
-                                               for s in seq_ids] or [np.empty(0, np.int64)]), self.device)
+        slots = upload_indices(np.concatenate([self._next_slots(s, T) for s in seq_ids] or [np.empty(0, np.int64)]),
+                               self.device)
         self.write_rows(seq_ids, keys.reshape(B * T, H, D), values.reshape(B * T, H, D), slots)
 
     def write_rows(self, seq_ids: Sequence[int], keys: torch.Tensor, values: torch.Tensor,

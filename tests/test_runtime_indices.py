@@ -25,6 +25,7 @@ def test_slots_past_int32_raise(monkeypatch):
     _, kv = _modules()
     monkeypatch.setattr(kv.PagedKVCache, "device", torch.device("cpu"))
     cache = object.__new__(kv.PagedKVCache)
+    cache.num_blocks = 2 ** 27 + 1
     cache.block_size, cache._pages, cache._len = 16, {0: [2 ** 27 - 1, 2 ** 27]}, {0: 0}
     assert cache.slot_mapping([0], 16)[-1] == 2 ** 31 - 1
     with pytest.raises(OverflowError, match="2147483648"):
