@@ -286,6 +286,16 @@ int memopt_paged_attention(const memopt_attn_desc *desc, void *stream);
  * on each device resolves the array's device address there. */
 int memopt_paged_attention_noalloc(const memopt_attn_desc *desc, void *stream);
 
+/* Diagnostics, no counterpart in the reference: the path that multi-query
+ * calls of the calling thread over INT4 pages and fp16 pools take (workspace
+ * query included). Both compute the same function; AUTO, the default, takes
+ * the one estimated to be faster. The others are for tests and measurements
+ * that need one of them at any size. */
+#define MEMOPT_PATH_AUTO   0
+#define MEMOPT_PATH_STAGED 1  /* K and V staged as fp16, then attended (csrc/prefill.hip) */
+#define MEMOPT_PATH_DIRECT 2  /* attended straight from the cache (csrc/direct.hip)       */
+int memopt_multi_query_path(int32_t path);
+
 #ifdef __cplusplus
 }
 #endif

@@ -39,7 +39,6 @@
 // adds up (a launch of its own: the partials' workspace may hold anything).
 #include <algorithm>
 #include <cmath>
-#include <cstdlib>
 
 #include "attention.hpp"
 #include "page_format.hpp"
@@ -683,10 +682,11 @@ static double grid_time(double n, double both, double ramp) {
   return fill * (x <= 2.0 ? 1.0 : (1.0 - ramp) * x / 2 + ramp * std::ceil(x / 2));
 }
 
+// (An environment variable in its place cost each call 1 us.)
+static thread_local int32_t t_path = MEMOPT_PATH_AUTO;
+
 static bool direct_faster(const memopt_attn_desc &d) {
-  // (MEMOPT_MULTI_QUERY_PATH=staged or =direct takes one path for every call,
-  // so that tests reach both at any size.)
-  if (const char *e = std::getenv("MEMOPT_MULTI_QUERY_PATH")) return *e == 'd';
+  if (t_path != MEMOPT_PATH_AUTO) return t_path == MEMOPT_PATH_DIRECT;
   const int64_t q = d.q_len, heads = (int64_t)d.num_heads * d.batch, tiles = (q + 127) / 128 * heads;
   if (q <= 128 || tiles <= 128) return true;
   // Pairs of one sequence at the longest context the block table holds.
@@ -837,3 +837,12 @@ int launch_direct(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hip
 }
 
 }  // namespace memopt
+
+using namespace memopt;
+
+extern "C" int memopt_multi_query_path(int32_t path) {
+  MEMOPT_REQUIRE(path == MEMOPT_PATH_AUTO || path == MEMOPT_PATH_STAGED || path == MEMOPT_PATH_DIRECT,
+                 MEMOPT_ERR_INVALID, "multi_query_path: unknown path");
+  t_path = path;
+  return MEMOPT_OK;
+}

@@ -20,6 +20,18 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a ROCm GPU (MI355X) and the built HIP library")
 
 
+@pytest.fixture
+def multi_query_path():
+    """Sets the multi-query path of this thread's calls: "staged", "direct" or "auto"."""
+    import memopt_C
+
+    def take(name):
+        memopt_C._check(memopt_C._lib.memopt_multi_query_path(["auto", "staged", "direct"].index(name)))
+
+    yield take
+    take("auto")
+
+
 @pytest.fixture(autouse=True)
 def _fresh_pool(request):
     """Every GPU test starts without a pool. init_pool keeps a live pool of

@@ -189,6 +189,36 @@ def test_multi_query_workspace_holds_the_splits(lib, fmt, H, D, q_len, tokens, s
     assert need.value == (q_len * H * splits * (D + 2) * 4 if splits else staged)
 
 
+def test_multi_query_path_is_checked_and_per_thread(lib):
+    """Unknown paths are refused; a path set on one thread is not another's."""
+    import threading
+    import memopt_C
+    d = memopt_C.AttnDesc()
+    d.query = d.out = d.key_cache = d.block_tables = d.context_lens = 256
+    d.batch, d.q_len, d.num_heads, d.head_dim = 1, 16, 1, 64
+    d.kv_format, d.block_size, d.num_kv_blocks = 1, 16, 1 << 22
+    d.max_blocks_per_seq, d.max_seq_len, d.window_size = 1 << 22, 1 << 26, 1 << 26  # no room for a staged copy
+    ws = lib.memopt_attention_workspace_size
+    ws.argtypes = [ctypes.POINTER(memopt_C.AttnDesc), ctypes.POINTER(ctypes.c_int64)]
+
+    def size():
+        need = ctypes.c_int64()
+        assert ws(ctypes.byref(d), ctypes.byref(need)) == OK
+        return need.value
+
+    try:
+        assert lib.memopt_multi_query_path(3) == ERR_INVALID and lib.memopt_multi_query_path(-1) == ERR_INVALID
+        direct = size()
+        assert direct > 0 and lib.memopt_multi_query_path(1) == OK and size() == 0
+        other = []
+        t = threading.Thread(target=lambda: other.append(size()))
+        t.start()
+        t.join()
+        assert other == [direct]
+    finally:
+        assert lib.memopt_multi_query_path(0) == OK
+
+
 @pytest.mark.parametrize("fmt,units,tokens,splits", [
     (1, 8, 1024, 1), (1, 8, 6000, 11), (1, 120, 6000, 4), (1, 128, 6000, 4), (1, 129, 6000, 6), (1, 160, 6000, 5),
     (1, 192, 6000, 4), (1, 255, 6000, 4), (1, 256, 6000, 2), (1, 511, 6000, 2), (1, 512, 6000, 1),

@@ -151,7 +151,7 @@ def test_direct_rows_non_finite_scores(D, scale, n):
     ("pages", 4, 12, 64, 1000, 500, 1 << 20, True, "direct"),
     ("fp16", 2, 8, 128, 1024, 128, 1 << 20, False, "direct"),
 ])
-def test_multi_query_path_by_estimate(layout, B, H, D, n, Lq, W, causal, path, monkeypatch):
+def test_multi_query_path_by_estimate(layout, B, H, D, n, Lq, W, causal, path, multi_query_path):
     """Calls far to either side of the line between the direct kernel and the
     staged path run the faster one (equal bits), and both agree."""
     g = torch.Generator(device=dev()).manual_seed(Lq)
@@ -166,11 +166,10 @@ def test_multi_query_path_by_estimate(layout, B, H, D, n, Lq, W, causal, path, m
     bt = torch.randperm(nb, generator=g, device=dev()).to(torch.int32).view(B, -1).contiguous()
     cl = torch.full((B,), n, dtype=torch.int32, device=dev())
     out = {}
-    for name in ("", "staged", "direct"):
-        if name:
-            monkeypatch.setenv("MEMOPT_MULTI_QUERY_PATH", name)
+    for name in ("auto", "staged", "direct"):
+        multi_query_path(name)
         out[name] = memopt_C.dynamic_sparse_attention(q, k, v, bt, cl, n, W, causal=causal)
-    assert torch.equal(out[""], out[path]) and not torch.equal(out["staged"], out["direct"])
+    assert torch.equal(out["auto"], out[path]) and not torch.equal(out["staged"], out["direct"])
     assert_close(out["direct"], out["staged"].cpu(), what="direct vs staged")
 
 

@@ -283,9 +283,8 @@ def test_config4_full_rows_int4_pages():
 
 
 def _prefill_with_env(env, *args, **kw):
-    """One attention call on the staged path with the given environment overrides in place."""
+    """One attention call with the given environment overrides in place."""
     import os
-    env = dict(env, MEMOPT_MULTI_QUERY_PATH="staged")
     old = {k: os.environ.get(k) for k in env}
     os.environ.update(env)
     try:
@@ -301,7 +300,7 @@ def _prefill_with_env(env, *args, **kw):
 
 
 @pytest.mark.parametrize("D,fmt", [(128, "int4"), (64, "int4"), (128, "fp16")])
-def test_in_kernel_staging_paths_agree(D, fmt):
+def test_in_kernel_staging_paths_agree(D, fmt, multi_query_path):
     """Long causal prefill (q_len 4096, so the attention kernel stages the
     workspace itself: each XCD's first (sequence, head) unit by a staging
     launch, every later unit by the first workgroups of the unit before it)
@@ -311,6 +310,7 @@ def test_in_kernel_staging_paths_agree(D, fmt):
     waiting workgroup stages its unit itself (MEMOPT_PREFILL_STAGE_SPIN=-1)
     agree, and sequence 0 matches fp32 attention over the dequantized pool
     on every row of two heads."""
+    multi_query_path("staged")  # (D = 64 takes the direct kernel by itself)
     B, S, H, W, sinks = 3, 4096, 8, 1024, 4
     torch.manual_seed(13)
     nbps = S // 16

@@ -18,5 +18,5 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(autouse=True)
-def _staged(monkeypatch):
-    monkeypatch.setenv("MEMOPT_MULTI_QUERY_PATH", "staged")
+def _staged(multi_query_path):
+    multi_query_path("staged")

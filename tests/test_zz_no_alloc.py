@@ -20,9 +20,9 @@ SCRATCH_BYTES = 4 << 20
 
 
 @pytest.fixture
-def staged(monkeypatch):
+def staged(multi_query_path):
     """Multi-query calls of these sizes take the direct kernel by themselves."""
-    monkeypatch.setenv("MEMOPT_MULTI_QUERY_PATH", "staged")
+    multi_query_path("staged")
 
 
 def _entry_points():
