@@ -86,10 +86,11 @@ def autochunk_prefill(cache: PagedKVCache, seq_id: int, query: torch.Tensor, key
         cache.reserve(seq_id, min(s1, rows) - min(s0, rows))  # raises at the first chunk past n_fit
         n = start + s1
         cache.write_rows([seq_id], keys[s0:s1], values[s0:s1], index.slots[s0:s1])
-        memopt_C.PreparedAttention(query[s0:s1].unsqueeze(0), k_pool, v_pool,
-                                   index.table[:, :pages_needed(n, cache.block_size)], index.lens[i:i + 1], n,
-                                   window_size, num_sink_tokens=num_sink_tokens, causal=True,
-                                   out=out[s0:s1].unsqueeze(0))()
+        with memopt_C._on(k_pool.device):  # (a plan launches on the current device)
+            memopt_C.PreparedAttention(query[s0:s1].unsqueeze(0), k_pool, v_pool,
+                                       index.table[:, :pages_needed(n, cache.block_size)], index.lens[i:i + 1], n,
+                                       window_size, num_sink_tokens=num_sink_tokens, causal=True,
+                                       out=out[s0:s1].unsqueeze(0))()
     return out
 
 

@@ -1,6 +1,9 @@
 """autochunk_prefill where the pool cannot hold the whole prompt: the chunks
 that fit are written and attended, then the call raises; and a shorter prompt
-appended after them. And where there are fewer key rows than queries."""
+appended after them. Where there are fewer key rows than queries. And every
+launch is made with the tensors' device current."""
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -53,3 +56,33 @@ def test_autochunk_fewer_keys_than_queries(held, rows):
                                                  held + s0 + C, 64, num_sink_tokens=4, causal=True)
         assert torch.equal(out[s0:s0 + C], want[0])
     assert len(cache.pages(0)) == len(cache.pages(1))
+
+
+def test_autochunk_launches_on_the_tensors_device(monkeypatch):
+    """The device guard (nothing to enter where the device is current already)
+    is held around every launch, so a cache on another GPU than the current
+    one launches there."""
+    import memopt_C as M
+    import memopt_runtime as R
+    held, launches = [], []
+
+    @contextlib.contextmanager
+    def on(device):
+        held.append(device)
+        yield
+        held.pop()
+
+    def guarded(name):
+        call = getattr(M, name)
+        monkeypatch.setattr(M, name, lambda *a: (launches.append((name, list(held))), call(*a))[1])
+
+    H, D, S = 2, 64, 50
+    q, k, v = (torch.randn(S, H, D, device=dev(), dtype=torch.float16) for _ in range(3))
+    cache = R.PagedKVCache(8, H, D, kv_format="int4")
+    cache.add_sequence(0)
+    monkeypatch.setattr(M, "_on", on)
+    guarded("_c_attn")
+    guarded("_c_write")
+    R.autochunk_prefill(cache, 0, q, k, v, chunk_tokens=20)
+    assert [n for n, _ in launches] == ["_c_write", "_c_attn"] * 3
+    assert all(devices[-1:] == [q.device] for _, devices in launches)
