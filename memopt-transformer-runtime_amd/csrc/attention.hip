@@ -10,10 +10,11 @@
 //   * fp16 cache, q_len == 1, pages of 16 * 2^k tokens, D in {64, 128},
 //     16-byte aligned rows -> decode_fp16 (split-K, HBM-streaming;
 //     decode_fp16.hip);
-//   * q_len >= 2, D in {64, 128}, pages of a multiple of 16 tokens: few
-//     queries, few query tiles, or token-major INT4 codes -> direct (fp16
-//     MFMA straight from the cache, split-K; direct.hip); other calls over
-//     fp16 pools or INT4 pages -> prefill (staged, fp16 MFMA; prefill.hip);
+//   * q_len >= 2, D in {64, 128}, pages of a multiple of 16 tokens:
+//     token-major INT4 codes, and calls that it runs faster by estimate
+//     -> direct (fp16 MFMA straight from the cache, split-K; direct.hip);
+//     other calls over fp16 pools or INT4 pages -> prefill (staged, fp16
+//     MFMA; prefill.hip);
 //   * anything else -> generic_attention_kernel below: one wave per
 //     (b, query, head), lanes over head dims, keys visited in order with an
 //     online softmax. INT4 elements are dequantized to fp16 exactly as the

@@ -87,7 +87,7 @@ unsigned long long next_decode_tag();
 // add after it counts, one round trip and no retry. (A compare-and-swap per
 // arrival, retried whenever another split got in between, cost about 2 us
 // per split: one sequence of 131072 tokens x 32 heads in 24 splits took
-// 139 us, with the add 97 us.) Two cases start elsewhere: a word above this
+// 146 us, with the add 97 us.) Two cases start elsewhere: a word above this
 // tag (an older launch replayed from a graph after newer ones, or foreign
 // data) is replaced by compare-and-swap, and a replay of the launch that
 // used the word last starts at the full count and ends at twice that, from
@@ -205,9 +205,9 @@ int64_t staged_copy_bytes(const memopt_attn_desc &d);  // the same, also past th
 int launch_prefill(const memopt_attn_desc &d, int32_t W, float qk_scale_log2, hipStream_t stream);
 
 // Multi-query kernel without staging (direct.hip): calls over INT4 pages and
-// fp16 pools with few queries or few query tiles, and any number of queries
-// over token-major INT4 codes (D in {64, 128}, pages of a multiple of 16
-// tokens, aligned strides).
+// fp16 pools that it is estimated to run faster than the staged path, and any
+// number of queries over token-major INT4 codes (D in {64, 128}, pages of a
+// multiple of 16 tokens, aligned strides).
 bool direct_supported(const memopt_attn_desc &d);
 // Bytes of split-K partials; a call that has less room runs fewer splits.
 int64_t direct_workspace_bytes(const memopt_attn_desc &d);
