@@ -583,6 +583,8 @@ static DecodeShape decode_shape() {
 //    of 12 splits in 8, and at most 0.88 on unequal lengths, in 4 0.80 and
 //    1.07; 66 units of 6000 tokens 39 us in 7, 51 in 4; 120 67 in 6, 68 in 4;
 //    160 units 0.90 and 1.02 of the time of 5 splits in 6, 0.96 and 1.20 in 3);
+//    where contexts are too short for two, up to a quarter of the CUs one
+//    workgroup per CU again (64 units of 2800 tokens 19 us in 4, 25 in 5);
 //  * 256 to 511 units: 2 (unsplit is up to 8 % faster on equal lengths, but
 //    10 % slower on lengths from a third to the whole of 4000 tokens);
 //  * at least 4 page batches per wave, and INT4 contexts of up to 64 pages are
@@ -600,7 +602,7 @@ int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool 
   else if (int4) s = 2 * units <= cus ? 2 * cus / units : (3 * cus + units - 1) / units;
   else s = 5 * units <= cus ? cus / units : std::max<int64_t>(6, 2 * cus / units);
   const int64_t cap = max_pages_visited / (4LL * sh.nw * sh.u);
-  if (s > cap) s = cap;
+  if (s > cap) s = !int4 && 4 * units <= cus ? std::min(cap, cus / units) : cap;
   if (int4 && max_pages_visited <= 64) s = 1;
   if (s < 1) s = 1;
   if (s > 64) s = 64;

@@ -222,7 +222,7 @@ def test_multi_query_path_is_checked_and_per_thread(lib):
 @pytest.mark.parametrize("fmt,units,tokens,splits", [
     (1, 8, 1024, 1), (1, 8, 6000, 11), (1, 120, 6000, 4), (1, 128, 6000, 4), (1, 129, 6000, 6), (1, 160, 6000, 5),
     (1, 192, 6000, 4), (1, 255, 6000, 4), (1, 256, 6000, 2), (1, 511, 6000, 2), (1, 512, 6000, 1),
-    (0, 40, 6000, 6), (0, 51, 6000, 5), (0, 52, 6000, 9), (0, 64, 6000, 8), (0, 96, 6000, 6), (0, 200, 6000, 6),
+    (0, 40, 6000, 6), (0, 51, 6000, 5), (0, 52, 6000, 9), (0, 64, 6000, 8), (0, 64, 2800, 4), (0, 60, 3500, 4), (0, 96, 6000, 6), (0, 200, 6000, 6),
     (0, 255, 6000, 6), (0, 256, 6000, 2), (0, 200, 1500, 2), (0, 200, 900, 1),
 ])
 def test_decode_split_counts(lib, fmt, units, tokens, splits):
