@@ -138,8 +138,8 @@ __global__ __launch_bounds__(NW * 64) void decode_int4_kernel(const DecodeParams
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // Head clusters (cluster_heads): grid (8 hc, groups, ceil(units / 8)) over
-  // the units u = (b, split), or (8 hc, 1, units * groups / 8) for fewer than
-  // 8 units. blockIdx.x is 8 * head of the cluster + XCD in both.
+  // the units u = (b, split), or (8 hc, 1, units * groups / 8) for a few units,
+  // not a multiple of 8. blockIdx.x is 8 * head of the cluster + XCD in both.
   int32_t b = blockIdx.z, h = blockIdx.y, split = blockIdx.x;
   if (p.hc > 1) {
     const int32_t xcd = blockIdx.x & 7;
@@ -626,22 +626,24 @@ int decode_splits(int32_t batch, int32_t heads, int32_t max_pages_visited, bool 
 // the mean of four random placements of three long ones among 32: 228, 190,
 // 168). A cluster's heads follow each other on their XCD: a stride between
 // them puts them on the same shader engine (62 us instead of 37 for the two
-// long ones of 16 x 12 heads of 64). Fewer than 8 units are clustered where
-// the clusters deal out evenly, and calls of fewer than 6000 blocks (16 tokens
-// of one head) not at all: the caches hold their lines, and finding its unit
-// costs a workgroup 0.1 to 0.5 us (16 sequences of 120 tokens x 40 heads of 128,
-// 5120 blocks: 11.4 us, clustered 11.6; 200 tokens x 32 heads, 6656 blocks:
-// 11.9 and 10.1; of 64, 16 x 20 heads, 5440 blocks 7.5 and 7.5, 8000 10.8 and
-// 8.5). With the double buffering, 16 sequences of 4096 tokens x 32 heads of
-// 128 (302 MB) went from 139 to 89 us, 8 heads of 64 from 20 to 13.5. What is left is throughput below the L1s: per page and
-// head the loads touch 64 pieces of lines (the page layout: 18), and neither
-// more pages in flight nor more waves changed it.
+// long ones of 16 x 12 heads of 64). Fewer than 64 units, not a multiple of
+// 8, are clustered so that the clusters deal out evenly (12 units of 40 heads
+// of 128 over 40000 tokens: 55 us in fours, 66 in eights), and calls of fewer
+// than 6000 blocks (16 tokens of one head) not at all: the caches hold their
+// lines, and finding its unit costs a workgroup 0.1 to 0.5 us (16 sequences of
+// 120 tokens x 40 heads of 128, 5120 blocks: 11.4 us, clustered 11.6; 200
+// tokens x 32 heads, 6656 blocks: 11.9 and 10.1; of 64, 16 x 20 heads, 5440
+// blocks 7.5 and 7.5, 8000 10.8 and 8.5). With the double buffering, 16
+// sequences of 4096 tokens x 32 heads of 128 (302 MB) went from 139 to 89 us,
+// 8 heads of 64 from 20 to 13.5. What is left is throughput below the L1s: per
+// page and head the loads touch 64 pieces of lines (the page layout: 18), and
+// neither more pages in flight nor more waves changed it.
 static int32_t cluster_heads(int64_t units, int32_t H, int32_t D, int64_t blocks) {
   if (blocks < 6000) return 1;
   const int32_t line = 256 / D;
   int32_t best = 1;
   for (int32_t hc = 2; hc <= 8 && hc <= H; ++hc) {
-    if (H % hc != 0 || (units < 8 && units * (H / hc) % 8 != 0)) continue;
+    if (H % hc != 0 || !(units % 8 == 0 || units >= 64 || units * (H / hc) % 8 == 0)) continue;
     if (hc % line == 0 || best % line != 0) best = hc;
   }
   return (units + 7) / 8 * (H / best) <= 65535 ? best : 1;  // (grid dimensions)
@@ -675,7 +677,7 @@ int launch_decode_int4(const DecodeParams &params, int32_t batch, int32_t D, int
   p.hc = p.pages ? 1 : cluster_heads(units, p.H, D, (int64_t)batch * p.H * pages);
   p.groups = p.H / p.hc;
   dim3 grid(p.splits, p.H, batch);
-  if (p.hc > 1 && units >= 8) grid = dim3(8 * p.hc, p.groups, (unsigned)((units + 7) / 8));
+  if (p.hc > 1 && (units % 8 == 0 || units >= 64)) grid = dim3(8 * p.hc, p.groups, (unsigned)((units + 7) / 8));
   else if (p.hc > 1) grid = dim3(8 * p.hc, 1, (unsigned)(units * p.groups / 8));
   if (D == 128 && scale_dtype == MEMOPT_SCALE_F16)
     launch_shape<128, half_t>(p, grid, sh, stream);
