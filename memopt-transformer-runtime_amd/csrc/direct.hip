@@ -647,33 +647,34 @@ static int direct_qb(const memopt_attn_desc &d) { return d.q_len <= 16 ? 1 : 2; 
 
 // Where the direct kernel beats the staged path (staging and attention
 // launches together). Both times are estimated, in us, from sums fitted to
-// both paths timed on 61000 random calls over pages and fp16 pools (1 to 40
+// both paths timed on 96000 random calls over pages and fp16 pools (1 to 40
 // heads, 1 to 16 sequences, 2 to 8192 queries, 20 to 32768 tokens, windows,
 // causal or not, equal and unequal lengths; median error 4 to 6 %):
 //  * a workgroup takes a fixed time and one per key it visits, and `both`
 //    more of that when a second one shares its CU; past two per CU the grid
-//    runs in rounds, whose last one counts `ramp` in full. A causal staged
-//    grid ends with its longest tile;
+//    runs in rounds, whose last one counts `ramp` in full (causal staged
+//    grids start their longest tiles first, which fills it);
+//  * a causal staged grid ends with its longest tile;
 //  * staging a (token, head, dim) of K and V costs `stage` per million;
-//  * each block of 32 queries reads its keys again: with many heads at once
-//    these reads pass the caches, at 150 / sqrt(MB of K and V) MB per us
-//    (16 sequences of 2277 fp16 tokens x 32 heads of 128, 486 queries: 1571
-//    us, staged 576; 178 queries on 3568 tokens x 32 heads of 64 525 and 371).
+//  * each block of 32 queries reads its keys again: from 256 heads on these
+//    reads leave the caches, at about 7 TB/s (16 sequences of 2277 fp16 tokens
+//    x 32 heads of 128, 486 queries: 1571 us, staged 576).
 // The estimates decide above 128 queries and 128 tiles (fewer tiles leave half
 // of the CUs idle on the staged path). Fixed numbers of queries, tiles and
 // (query, key) pairs, which drew the line before, lost 8 to 45 % on 266 of
-// those calls (4 x 4 heads of 128, 3540 queries in a 512-token window, not
+// 61500 calls (4 x 4 heads of 128, 3540 queries in a 512-token window, not
 // causal: 50 us, staged 40; 1 x 32 heads, fp16, 1687 causal queries: 51 and
-// 44; 2 x 40 heads, 530 queries: 49 and 43); on 34900 further random calls
-// this rule loses more than 8 % on 31.
+// 44; 2 x 40 heads, 530 queries: 49 and 43). On 31300 further random calls
+// this rule takes a path more than 8 % slower than the staged one 41 times,
+// and one more than 15 % slower than the better one 97 times.
 struct PathCost {
   double block, key, both;       // direct: per block, per thousand keys
   double tile, tile_key, tile_both, stage;
 };
 static const PathCost kPathCost[2][2] = {
     // D = 64, 128
-    {{1.4, 6.2, 0.39, 2.4, 21.5, 0.30, 0.84}, {2.7, 7.2, 0.87, 6.6, 25.3, 0.42, 0.70}},  // pages
-    {{1.3, 7.5, 0.41, 2.4, 21.5, 0.30, 1.16}, {1.9, 8.1, 1.18, 6.6, 25.3, 0.42, 0.92}},  // fp16 pools
+    {{1.3, 6.2, 0.37, 2.4, 21.0, 0.285, 0.94}, {2.7, 7.3, 0.85, 6.4, 24.6, 0.42, 0.76}},   // pages
+    {{1.3, 7.3, 0.46, 2.4, 21.0, 0.285, 1.33}, {1.95, 8.1, 1.18, 6.4, 24.6, 0.42, 1.01}},  // fp16 pools
 };
 
 // Time of n equal workgroups in units of one alone on its CU.
@@ -706,12 +707,15 @@ static bool direct_faster(const memopt_attn_desc &d) {
   const double longest = 1e-3 * (double)(d.causal ? std::min(T, W + 127) : W);
   const double blocks = (double)((q + 31) / 32);
   const double melems = 1e-6 * (double)(std::min(T, d.causal ? q + W : W) * heads * d.head_dim);  // K and V staged
-  double direct = 4.5 + (c.block + c.key * keys) * grid_time(blocks * heads, c.both, 0.42);
-  const double staged = 10.0 + (c.tile + c.tile_key * tile_keys) * grid_time((double)tiles, c.tile_both, 0.22) +
-                        16.5 * (longest - tile_keys) + c.stage * melems;
-  const double passes = blocks * std::min(1.0, heads / 128.0), mb = melems * (pages ? 1.125 : 4.0);
-  if (passes > 1.0) direct = std::max(direct, passes * mb * std::sqrt(mb) / 150.0);
-  return direct < 0.94 * staged;
+  const double staged = 10.0 + 17.7 * (longest - tile_keys) + c.stage * melems +
+                        (c.tile + c.tile_key * tile_keys) *
+                            grid_time((double)tiles, c.tile_both, d.causal ? 0.08 : 0.65);
+  const double compute = 4.5 + (c.block + c.key * keys) * grid_time(blocks * heads, c.both, 0.42);
+  // MB that the blocks of all heads read at once, and how often
+  const double mb = 1e-3 * keys * heads * d.head_dim * (pages ? 1.125 : 4.0);
+  const double passes = blocks * std::min(1.0, heads / 256.0);
+  const double direct = std::max(compute, passes > 1.0 ? passes * mb / 7.0 : 0.0);
+  return direct < 0.95 * staged;
 }
 
 static int64_t direct_query_blocks(const memopt_attn_desc &d) {
