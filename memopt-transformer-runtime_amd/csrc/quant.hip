@@ -242,21 +242,23 @@ __global__ __launch_bounds__(kThreads) void write_int4_kernel(
 //    rate of this mix is 5.2; 6000-token prompts, all aligned, 90).
 //  * The other tokens of the group (decode appends, ragged heads and tails,
 //    arbitrary slots) scatter 8-element chunks like write_int4_kernel.
-// `starts`: the lanes whose token may start a page. Below 1.5 M elements of K
-// only lane 15's, the group's first, may: a page at another token is loaded
-// after the slot check and the rest of its group scatters after that, which
-// in a launch that lasts one memory round trip takes longer than scattering
-// the group at once (100 tokens x 8 heads of 64 from token 5 of a page on: 3.7
-// us scattered, 4.2 with pages; 512 x 20 heads of 64, 0.66 M, 4.0 and 4.4; 512
-// x 32 of 128, 2.1 M, 5.7 and 5.35; 5000 x 8 of 64, 2.6 M, 6.1 and 5.4).
+// `runs`: pages may start at any token, from 1.5 M elements of K on; below
+// that only at a group's first: a page at another token is loaded after the
+// slot check and the rest of its group scatters after that, which in a launch
+// that lasts one memory round trip takes longer than scattering the group at
+// once (100 tokens x 8 heads of 64 from token 5 of a page on: 3.7 us scattered,
+// 4.2 with pages; 512 x 20 heads of 64, 0.66 M, 4.0 and 4.4; 512 x 32 of 128,
+// 2.1 M, 5.7 and 5.35; 5000 x 8 of 64, 2.6 M, 6.1 and 5.4).
 // A wave finds both from the slots of its tokens, the 15 before and the 16
 // after, with a few scalar steps on a ballot, so all waves agree on which
-// tokens are part of a page.
+// tokens are part of a page; a group that is one page by itself needs only its
+// own (the steps made aligned writes of 24020 tokens x 20 heads of 64 29.6 us
+// instead of 28.4).
 // 32-bit indexing: requires T * H * D < 2^31 (checked by the caller).
 template <int D>
 __global__ __launch_bounds__(kThreads) void write_int4_pages_kernel(
     const half_t *__restrict__ keys, const half_t *__restrict__ values, uint8_t *__restrict__ pool,
-    const int32_t *__restrict__ slots, uint32_t T, uint32_t H, int64_t n_slots, uint64_t starts) {
+    const int32_t *__restrict__ slots, uint32_t T, uint32_t H, int64_t n_slots, bool runs) {
   constexpr int DPL = D / 8;    // dims per lane per token in the page layout
   constexpr int GL = 64 / DPL;  // lanes per 64-group
   constexpr int CPR = D / 8;    // 8-element chunks per (token, head) row
@@ -290,20 +292,29 @@ __global__ __launch_bounds__(kThreads) void write_int4_pages_kernel(
   const int32_t tok = (int32_t)(t0 + lane) - 15;
   const bool in = lane < 47 && tok >= 0 && tok < (int32_t)T;
   const int32_t sl = in ? slots[tok] : -2;
-  const int32_t nxt = __shfl_down(sl, 1, 64);
-  uint64_t run = __ballot(in && lane < 46 && nxt == sl + 1);  // token i + 1 follows token i
-  run &= run >> 1;
-  run &= run >> 2;
-  run &= run >> 4;
-  run &= run >> 7;  // the 15 tokens after token i follow it
-  const uint64_t start = run & starts & __ballot(sl >= 0 && (sl & 15) == 0 && (int64_t)sl + 16 <= n_slots);
-  const uint32_t own = (uint32_t)(start >> 15) & 0xFFFFu;  // a page starting in this group (at most one)
-  uint64_t cov = start;
-  cov |= cov << 1;
-  cov |= cov << 2;
-  cov |= cov << 4;
-  cov |= cov << 8;
-  const uint32_t paged = (uint32_t)(cov >> 15) & 0xFFFFu;  // tokens of the group that are part of a page
+  uint32_t own = 0;    // a page starting in this group (at most one)
+  uint32_t paged = 0;  // tokens of the group that are part of a page
+  const int32_t sg = __builtin_amdgcn_readlane(sl, 15);
+  if (__all(lane < 15 || lane > 30 || sl == sg + (int32_t)lane - 15) && sg >= 0 && (sg & 15) == 0 &&
+      (int64_t)sg + 16 <= n_slots) {  // the group is a page
+    own = 1;
+    paged = 0xFFFFu;
+  } else if (runs) {
+    const int32_t nxt = __shfl_down(sl, 1, 64);
+    uint64_t run = __ballot(in && lane < 46 && nxt == sl + 1);  // token i + 1 follows token i
+    run &= run >> 1;
+    run &= run >> 2;
+    run &= run >> 4;
+    run &= run >> 7;  // the 15 tokens after token i follow it
+    const uint64_t start = run & __ballot(sl >= 0 && (sl & 15) == 0 && (int64_t)sl + 16 <= n_slots);
+    own = (uint32_t)(start >> 15) & 0xFFFFu;
+    uint64_t cov = start;
+    cov |= cov << 1;
+    cov |= cov << 2;
+    cov |= cov << 4;
+    cov |= cov << 8;
+    paged = (uint32_t)(cov >> 15) & 0xFFFFu;
+  }
 
   if (own != 0) {
     const uint32_t off = __builtin_ctz(own);  // wave-uniform
@@ -535,15 +546,15 @@ int memopt_write_cache(const void *keys, const void *values, int64_t num_tokens,
     const int64_t waves = (num_tokens + 15) / 16 * num_heads * 2;
     if (vec && waves < (1LL << 32) && num_tokens < (1LL << 31) && (head_dim == 64 || head_dim == 128)) {
       const unsigned grid = (unsigned)((waves + kThreads / 64 - 1) / (kThreads / 64));
-      const uint64_t starts = num_tokens * row < 1500000 ? 1ull << 15 : ~0ull;
+      const bool runs = num_tokens * row >= 1500000;
       if (head_dim == 128)
         hipLaunchKernelGGL(write_int4_pages_kernel<128>, dim3(grid), dim3(kThreads), 0, s, (const half_t *)keys,
                            (const half_t *)values, (uint8_t *)p.key, slot_mapping, (uint32_t)num_tokens,
-                           (uint32_t)num_heads, n_slots, starts);
+                           (uint32_t)num_heads, n_slots, runs);
       else
         hipLaunchKernelGGL(write_int4_pages_kernel<64>, dim3(grid), dim3(kThreads), 0, s, (const half_t *)keys,
                            (const half_t *)values, (uint8_t *)p.key, slot_mapping, (uint32_t)num_tokens,
-                           (uint32_t)num_heads, n_slots, starts);
+                           (uint32_t)num_heads, n_slots, runs);
     } else if (vec)
       hipLaunchKernelGGL(write_int4_kernel<true>, dim3(grid_for(n)), dim3(kThreads), 0, s,
                          (const half_t *)keys, (const half_t *)values, (uint8_t *)p.key, slot_mapping, n,
