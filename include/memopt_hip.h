@@ -226,8 +226,8 @@ int memopt_dynamic_sparse_attention(const void *query, int32_t batch, int32_t q_
  * `workspace` (device, >= memopt_attention_workspace_size bytes) holds the
  * decode's split-K partials and arrival counters, or a multi-query call's
  * staged K/V and staging flags or split partials; it may be NULL when that
- * size is 0 (and for multi-query calls over token-major INT4 codes, which
- * then run unsplit). A decode
+ * size is 0 (and for multi-query calls that attend straight from the cache,
+ * which then run unsplit). A decode
  * (q_len == 1) workspace must be zero before its first use; later calls may
  * reuse it without clearing (each call's counters carry the call's id, so
  * what an earlier call left is never taken for its own). A multi-query

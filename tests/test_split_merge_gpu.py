@@ -92,20 +92,19 @@ def test_token_major_head_clusters(B, H):
 
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("B,H,splits", [(1, 16, 1), (3, 32, 1), (2, 20, 2), (7, 8, 1), (8, 3, 1), (9, 12, 1),
-                                        (5, 7, 3), (16, 40, 1), (1, 64, 8), (2, 1, 5)])
+                                        (5, 7, 3), (16, 40, 1), (1, 64, 8), (2, 1, 5), (12, 40, 1), (12, 10, 1),
+                                        (11, 4, 6)])
 def test_token_major_head_clusters_of_long_calls(B, H, splits, D, monkeypatch):
     """Calls whose block tables hold enough pages for head clusters (most of
-    them unlinked here): fewer than 8 (sequence, split) units, 8, numbers
-    between multiples of 8; cluster sizes 1 to 8, one to eight per unit."""
+    them unlinked here): fewer than 8 (sequence, split) units, 8, few and many
+    between multiples of 8; cluster sizes 1 to 8, one to ten per unit."""
     monkeypatch.setenv("MEMOPT_DECODE_SPLITS", str(splits))
     rng = np.random.default_rng(B * 100 + H)
     ctx = [int(x) for x in rng.integers(1, 90, B)]
     q, k, v, bt, cl = _case(B + H, B, H, D, ctx)
     M = 6000 // (B * H) + 2
     wide = np.full((B, M), -1, np.int32)
-    at = 7 * np.arange(bt.shape[1]) % M                # pages spread over the table, so over the splits
-    assert len(set(at)) == bt.shape[1]
-    at.sort()
+    at = np.sort(rng.permutation(M)[:bt.shape[1]])     # pages spread over the table, so over the splits
     wide[:, at] = bt
     cl = np.array([16 * int(at[(c - 1) // 16]) + (c - 1) % 16 + 1 for c in ctx], np.int32)
     (kq, ks), (vq, vs) = O.quantize_int4(k), O.quantize_int4(v)
